@@ -684,6 +684,9 @@ int link_view(const nq_gauge* gc, int lk, LinkView* v)
   v->prec = lk;
   v->data[0] = b.p;
   v->data[1] = (const char*)b.p + per;
+  v->unit = 0;
+  for (int mu = 0; mu < 4; mu++)
+    if (std::fabs(g->det[mu][0] - 1) < 1e-13 && std::fabs(g->det[mu][1]) < 1e-13) v->unit |= 1u << mu;
   for (int p = 0; p < 2; p++)
     for (int mu = 0; mu < 4; mu++) {
       v->det[p][2 * mu][0] = g->det[mu][0];

@@ -45,6 +45,15 @@ __device__ __forceinline__ void fma_to(cx<R>& acc, cx<R> a, cx<R> b)
   acc.im = fma(a.im, b.re, acc.im);
 }
 
+// A uniform value that no workgroup of the launch writes, read through the constant
+// address space: a scalar load, which does not queue behind the vector loads in flight
+// (vmcnt counts in order; a vector load's wait would drain every prefetch before it)
+template <class T>
+__device__ __forceinline__ T sload(const T* p)
+{
+  return *(const __attribute__((address_space(4))) T*)(uintptr_t)p;
+}
+
 // ---------------------------------------------------------------- geometry
 struct Site {
   int t, x, y, z, th, tl, xt, xi, yt, yi;
@@ -311,7 +320,10 @@ struct SpAcc {
     if constexpr (SP == SP_F16) {
       float m = 0.f;
 #pragma unroll
-      for (int k = 0; k < NC; k++) m = fmaxf(m, fmaxf(fabsf((float)s[k].re), fabsf((float)s[k].im)));
+      for (int k = 0; k < NC; k++) {
+        const float a = (float)s[k].re, b = (float)s[k].im;
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a), "v"(b));
+      }
       // sites whose largest component is below 1e-30 are stored as zero: 1/m would
       // overflow for denormal m (fields far from a point source decay that far)
       if (!(m >= 1e-30f)) m = 0.f;
@@ -321,6 +333,26 @@ struct SpAcc {
     } else {
       store_packed<EB, NC, CP, R>(base, stride, e, s);
     }
+  }
+};
+
+// One FP16 spinor as stored: three records of four complex halves (component k is
+// halves 2(k%4), 2(k%4)+1 of record k/4) and the site's norm.
+struct RawF16 {
+  nq_u4 u[3];
+  float norm;
+  __device__ __forceinline__ void load(const SpinorView& v, int64_t stride, uint32_t e, int r)
+  {
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc((const char*)v.data + (int64_t)r * v.rstride * 4, 48 * stride);
+#pragma unroll
+    for (int q = 0; q < 3; q++) u[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, e * 16u, (uint32_t)(q * stride * 16), 0);
+    norm = bload_f1(make_rsrc(v.norm + (int64_t)r * stride, stride * 4), e * 4, 0);
+  }
+  // component k as the two converted halves
+  __device__ __forceinline__ cx<float> at(int k) const
+  {
+    const nq_hv8 h = __builtin_bit_cast(nq_hv8, u[k / 4]);
+    return mk<float>((float)h[2 * (k % 4)], (float)h[2 * (k % 4) + 1]);
   }
 };
 
@@ -359,7 +391,13 @@ struct Stage {
       ((float*)(lds + NG * kStageSites * 16))[t] = n;
     }
   }
-  // site at offset d (< kStageSites) of the staged range
+  // site at offset d (< kStageSites) of the staged range, FP16 records as stored
+  __device__ __forceinline__ static void get_raw(const char* lds, int d, RawF16& w)
+  {
+#pragma unroll
+    for (int q = 0; q < NG; q++) w.u[q] = *(const nq_u4*)(lds + (q * kStageSites + d) * 16);
+    w.norm = ((const float*)(lds + NG * kStageSites * 16))[d];
+  }
   template <class R>
   __device__ __forceinline__ static void get(const char* lds, int d, cx<R> s[NC])
   {
@@ -384,20 +422,40 @@ template <int LK, class R, int CP = kLinkCP>
 struct LkAcc {
   static constexpr int NC = lk_nc(LK);
   static constexpr int EB = lk_eb(LK);
-  // U as u[3][3]; slot s is a packed array of NC elements at base + s*NC*stride*EB bytes
+  // U as u[3][3]; slot s is a packed array of NC elements at base + s*NC*stride*EB bytes;
+  // unit: the slot's det is 1 (LinkView::unit), its product is left out
   __device__ __forceinline__ static void load(const void* base, int64_t stride, int slot, uint32_t e,
-                                              const double* det, cx<R> u[9])
+                                              const double* det, cx<R> u[9], bool unit = false)
+  {
+    load_stored(base, stride, slot, e, u);
+    complete(det, u, unit);
+  }
+  // the stored elements only
+  __device__ __forceinline__ static void load_stored(const void* base, int64_t stride, int slot, uint32_t e, cx<R>* u)
   {
     const char* sb = (const char*)base + (int64_t)slot * NC * stride * EB;
     load_packed<EB, NC, CP, R>(sb, (int64_t)NC * stride * EB, stride, e, u);
+  }
+  // row 2 = det * conj(row0 x row1) of a 12-real link
+  __device__ __forceinline__ static void complete(const double* det, cx<R> u[9], bool unit)
+  {
+    if constexpr (EB == 4) {
+      // widened once: left to itself the compiler reads the halves in every product
+      // (v_fma_mix_f32), which runs at half the rate of v_fma_f32
+#pragma unroll
+      for (int k = 0; k < NC; k++) asm("" : "+v"(u[k].re), "+v"(u[k].im));
+    }
     if constexpr (NC == 6) {
-      // row 2 = det * conj(row0 x row1)
-      const cx<R> dt = mk<R>((R)det[0], (R)det[1]);
 #pragma unroll
       for (int j = 0; j < 3; j++) {
         const int a = (j + 1) % 3, b = (j + 2) % 3;
-        const cx<R> c = u[a] * u[3 + b] - u[b] * u[3 + a];
-        u[6 + j] = dt * conjg(c);
+        const cx<R> p = u[a] * u[3 + b], q = u[b] * u[3 + a];
+        u[6 + j] = mk<R>(p.re - q.re, q.im - p.im);
+      }
+      if (!unit) {  // uniform over the launch
+        const cx<R> dt = mk<R>((R)det[0], (R)det[1]);
+#pragma unroll
+        for (int j = 0; j < 3; j++) u[6 + j] = dt * u[6 + j];
       }
     }
   }

@@ -89,6 +89,9 @@ struct LinkView {
   const void* data[2] = {nullptr, nullptr};  // indexed by output parity
   int prec = LK_F64_18;
   double det[2][8][2] = {};                  // [out parity][slot][re,im]
+  // bit mu: |det(U_mu) - 1| < 1e-13, the links of direction mu carry no phase.  The FP32
+  // and FP16 link kernels then leave out the product with det, which is 1 in FP32
+  unsigned unit = 0;
 };
 
 // Solver state living in device memory; updated by the finalisation kernel
