@@ -246,21 +246,20 @@ Geo make_geo(int T, int LX, int LY, int LZ, int tbmax, int tx, int ty)
   auto lg = [](int v) { int l = 0; while ((1 << l) < v) l++; return l; };
   g.TX = tx; g.logTX = lg(tx); g.NXT = LX / tx;
   g.TY = ty; g.logTY = lg(ty); g.NYT = LY / ty;
-  g.Sz = g.TB;
-  g.Syi = (int64_t)g.TB * LZ;
+  // pairs of z rows: with the 4 x 2 patch, 256 consecutive sites of a 64-slice t tile are
+  // a 2 x 2 x 2 cell of rows (NQ_ZTILE overrides; a power of two up to 16)
+  int tz = 2;
+  if (const char* ez = getenv("NQ_ZTILE")) tz = atoi(ez);
+  if (!pow2(tz)) tz = 1;
+  while (LZ % tz) tz /= 2;
+  g.TZ = tz; g.logTZ = lg(tz); g.NZT = LZ / tz;
+  g.Szi = g.TB;
+  g.Syi = g.Szi * g.TZ;
   g.Sxi = g.Syi * g.TY;
-  g.Syt = g.Sxi * g.TX;
+  g.Szt = g.Sxi * g.TX;
+  g.Syt = g.Szt * g.NZT;
   g.Sxt = g.Syt * g.NYT;
   g.Sth = g.Sxt * g.NXT;
-  // z-slab visit order of the batched kernels when every column is a whole number
-  // (at least two) of 256-site blocks; NQ_RB_ORDER=0 keeps the storage order
-  const int64_t col = (int64_t)g.TB * LZ / 2;
-  const char* ro = getenv("NQ_RB_ORDER");
-  const bool slabs = !(ro && ro[0] == '0');
-  if (slabs && g.Vh % 256 == 0 && col % 256 == 0 && col >= 512) {
-    g.rb_bpc = col / 256;
-    g.rb_ncol = g.Vh / col;
-  }
   return g;
 }
 

@@ -56,7 +56,7 @@ __device__ __forceinline__ T sload(const T* p)
 
 // ---------------------------------------------------------------- geometry
 struct Site {
-  int t, x, y, z, th, tl, xt, xi, yt, yi;
+  int t, x, y, z, th, tl, xt, xi, yt, yi, zt, zi;
   uint32_t dlx;  // rank in the device site order
 };
 
@@ -66,12 +66,14 @@ __device__ __forceinline__ Site site_of(const Geo& g, int par, uint32_t e)
   const uint32_t q = 2u * e;
   uint32_t r = q / (uint32_t)g.TB;
   const int tl0 = (int)(q - r * (uint32_t)g.TB);
-  const uint32_t r1 = r / (uint32_t)g.LZ;
-  s.z = (int)(r - r1 * (uint32_t)g.LZ);
-  s.yi = (int)(r1 & (uint32_t)(g.TY - 1));
-  const uint32_t r2 = r1 >> g.logTY;
-  s.xi = (int)(r2 & (uint32_t)(g.TX - 1));
-  const uint32_t r3 = r2 >> g.logTX;
+  s.zi = (int)(r & (uint32_t)(g.TZ - 1));
+  r >>= g.logTZ;
+  s.yi = (int)(r & (uint32_t)(g.TY - 1));
+  r >>= g.logTY;
+  s.xi = (int)(r & (uint32_t)(g.TX - 1));
+  r >>= g.logTX;
+  const uint32_t r3 = r / (uint32_t)g.NZT;
+  s.zt = (int)(r - r3 * (uint32_t)g.NZT);
   const uint32_t r4 = r3 / (uint32_t)g.NYT;
   s.yt = (int)(r3 - r4 * (uint32_t)g.NYT);
   const uint32_t r5 = r4 / (uint32_t)g.NXT;
@@ -79,6 +81,7 @@ __device__ __forceinline__ Site site_of(const Geo& g, int par, uint32_t e)
   s.th = (int)r5;
   s.x = s.xt * g.TX + s.xi;
   s.y = s.yt * g.TY + s.yi;
+  s.z = s.zt * g.TZ + s.zi;
   const int b = (par + tl0 + s.x + s.y + s.z) & 1;
   s.tl = tl0 + b;
   s.t = s.th * g.TB + s.tl;
@@ -110,7 +113,8 @@ __device__ __forceinline__ uint32_t neigh_eo(const Geo& g, const Site& s, int mu
     else d += s.yi > 0 ? -g.Syi : (int64_t)(g.TY - 1) * g.Syi + (s.yt == 0 ? (int64_t)(g.NYT - 1) * g.Syt : -g.Syt);
     break;
   default:
-    d += up ? (s.z == g.LZ - 1 ? -(int64_t)(g.LZ - 1) * g.Sz : g.Sz) : (s.z == 0 ? (int64_t)(g.LZ - 1) * g.Sz : -g.Sz);
+    if (up) d += s.zi < g.TZ - 1 ? g.Szi : -(int64_t)(g.TZ - 1) * g.Szi + (s.zt == g.NZT - 1 ? -(int64_t)(g.NZT - 1) * g.Szt : g.Szt);
+    else d += s.zi > 0 ? -g.Szi : (int64_t)(g.TZ - 1) * g.Szi + (s.zt == 0 ? (int64_t)(g.NZT - 1) * g.Szt : -g.Szt);
     break;
   }
   return (uint32_t)(d >> 1);
@@ -601,40 +605,6 @@ __device__ __forceinline__ Map map_thread_lb(const Shape& S, int64_t Vh, int64_t
 }
 
 __device__ __forceinline__ Map map_thread(const Shape& S, int64_t Vh) { return map_thread_lb(S, Vh, xcd_block()); }
-
-// Thread mapping of the register-blocked (multi-RHS) kernels (Shape W = 4, NRB = 1):
-// with g.rb_bpc > 0 the 256-site blocks are visited z slab by z slab, logical block
-// l -> slab l / rb_ncol and column l % rb_ncol -> stored block column * rb_bpc + slab.
-// A batched hop moves several times the bytes per site of a one-RHS hop, so in the
-// storage order the neighbour rows a y tile away (thousands of sites) have left the
-// XCD's L2 when they are read again; inside a slab the +-x and +-y neighbour blocks
-// of a block are a few blocks apart in the visit order.  Each (right-hand side,
-// chunk) pair is computed as in the storage order, so results do not change.
-__device__ __forceinline__ Map map_thread_rb(const Shape& S, const Geo& g, int nr)
-{
-  Map m;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int64_t lb = xcd_block();
-  const int rg = (int)(lb % S.NRG);
-  int64_t blk = lb / S.NRG;
-  if (g.rb_bpc > 0 && S.W == 4 && nr > 1) {  // one right-hand side: storage order
-    const int64_t zb = blk / g.rb_ncol, col = blk - zb * g.rb_ncol;
-    blk = col * g.rb_bpc + zb;
-  }
-  m.r = rg * S.NRB + wave % S.NRB;
-  m.chunk = blk * S.W + wave / S.NRB;
-  if (m.r >= S.NR) {
-    m.r = S.NR - 1;
-    m.chunk = INT64_MAX / 128;
-    m.e = 0;
-    m.active = false;
-    return m;
-  }
-  const int64_t e = m.chunk * 64 + lane;
-  m.active = e < g.Vh;
-  m.e = (uint32_t)e;
-  return m;
-}
 
 // Deterministic reductions over 64-site chunks.  Every wavefront holds the
 // partial of one (right-hand side r, chunk c) pair and stores it at

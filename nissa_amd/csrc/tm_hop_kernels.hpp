@@ -543,18 +543,21 @@ __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out
                                                    int64_t nchunks, double* partial)
 {
   using R = RealOf<SP>;
-  const Map m = map_thread_rb(S, g, nr);
+  const Map m = map_thread(S, g.Vh);
   const int r0 = m.r * RB, nrb = min(RB, nr - r0);
   unsigned busy = 0;
 #pragma unroll
   for (int b = 0; b < RB; b++)
     if (b < nrb && !(epi.st && rhs_idle(epi.st + r0 + b, epi.pred_reliable))) busy |= 1u << b;
   // right-hand sides that idle here are skipped by the finalisation as well.
-  // FP16: the busy right-hand sides' records of the workgroup's 256 sites are
-  // staged in LDS and the neighbours inside that range read from there (the
-  // batched hop is bound by the L2->L1 path: 12 sources, 684 -> 667 us for the
-  // plain hop and 987 -> 937 us for the CG tail at 32^3x64)
-  constexpr bool STG = SP == SP_F16;
+  // The busy right-hand sides' records of the workgroup's 256 sites are staged in LDS and
+  // the neighbours among those sites read from there, as far as the LDS holds two
+  // workgroups or more (FP16 any RB, FP32 up to two, FP64 one right-hand side per
+  // wavefront).  The batched hop is bound by the L2->L1 path: twelve right-hand sides at
+  // 24^3x48, FP64 825 -> 713 us, FP32 400 -> 308.  On lattices of a few dozen blocks the
+  // staging round trip only adds latency (16x8^3, FP32: 8.0 -> 9.2 us), so they skip it.
+  constexpr bool STG = SP == SP_F16 || (SP == SP_F32 && RB <= 2) || (SP == SP_F64 && RB == 1);
+  const bool stage = STG && g.Vh >= 64 * kStageSites;
   __shared__ __attribute__((aligned(16))) char lds[STG ? RB * Stage<SP, 12>::BYTES : 16];
   const uint32_t e0 = (uint32_t)((m.chunk - (threadIdx.x >> 6)) * 64);
   if (!busy) {  // uniform over the workgroup (one right-hand-side group)
@@ -565,7 +568,7 @@ __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out
     }
     return;
   }
-  if constexpr (STG) {
+  if (stage) {  // uniform over the launch
 #pragma unroll
     for (int b = 0; b < RB; b++)
       if (b < nrb && ((busy >> b) & 1u))
@@ -573,7 +576,7 @@ __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out
                            e0 + threadIdx.x < (uint64_t)g.Vh, (int)threadIdx.x, r0 + b);
     __syncthreads();
   }
-  const char* lp = STG ? lds : nullptr;
+  const char* lp = stage ? lds : nullptr;
   const uint32_t e = m.e;
   cx<R> o[RB][12];
 #pragma unroll
@@ -653,7 +656,7 @@ __global__ void __launch_bounds__(256, 2) k_tm_hop_rl(Geo g, int op, SpinorView 
                                                       double anis_d, int use_anis, HopEpi epi, Shape S, int nr,
                                                       int rpw, int64_t nchunks, double* partial)
 {
-  const Map m = map_thread_rb(S, g, nr);
+  const Map m = map_thread(S, g.Vh);
   const int r0 = m.r * rpw, r1 = min(r0 + rpw, nr);
   unsigned busy = 0;
   for (int r = r0; r < r1; r++) {

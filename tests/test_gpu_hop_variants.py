@@ -1,0 +1,71 @@
+"""Variants of the twisted-mass hop kernels at the sizes where their dispatch changes.
+
+* The batched FP16 hop keeps the links of a site in registers and loops over its
+  right-hand sides, in one or several groups; one or two right-hand sides on a large
+  lattice run the register-blocked kernel instead.  A source has the same bits alone and
+  in a batch whichever kernel and grouping the batch size picks, and small lattices agree
+  with the oracle (1e-10, the bar of the other mixed solves at residue 1e-24).
+* Links with a phase in every direction (the det of each slot enters the third row) and
+  with a phase in t alone (it is left out elsewhere).
+* Site orders whose z tile does not fit the extent (2 mod 4) or spans it.
+"""
+import numpy as np
+import pytest
+
+import nissa_amd as nq
+from helpers import gauss_eo, rel_l2
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def conf_of(L, seed, theta):
+    conf = nq.gauge_random_lx(L, seed, 0.3)
+    nq.gauge_phase_lx(L, conf, theta)
+    return conf
+
+
+# the largest has 262144 sites per parity, where one right-hand side runs another kernel
+# than three; 16^3x32 splits five right-hand sides into two groups
+@pytest.mark.parametrize("L,nr", [((32, 16, 16, 16), 5), ((16, 32, 32, 32), 3)])
+@pytest.mark.parametrize("prec", ["f16", "f16h"])
+def test_batched_f16_same_bits_alone(L, nr, prec):
+    conf = conf_of(L, 51, [1.0, 0, 0, 0])
+    with nq.Ctx(L) as ctx:
+        g = nq.Gauge(ctx, lx=conf)
+        src = [ctx.field(nq.SPINCOLOR, nq.LX, nq.source_lx(L, 60 + i)) for i in range(nr)]
+        sol = [ctx.field(nq.SPINCOLOR, nq.LX) for _ in range(nr)]
+        mus = [0.02 + 0.01 * i for i in range(nr)]
+        res = nq.tm_solve_eoprec_multi(ctx, g, 0.16, mus, 1000, 1e-14, sol, src, prec=prec)
+        assert all(r["rc"] == nq.NQ_OK and r["rel_res_sq"] < 2e-14 for r in res), res
+        for i in (0, nr - 1):
+            one = [ctx.field(nq.SPINCOLOR, nq.LX)]
+            nq.tm_solve_eoprec_multi(ctx, g, 0.16, mus[i:i + 1], 1000, 1e-14, one, src[i:i + 1], prec=prec)
+            assert np.array_equal(one[0].download(), sol[i].download()), i
+
+
+@pytest.mark.parametrize("L", [(10, 4, 2, 2), (4, 6, 4, 10), (8, 4, 4, 12)])
+@pytest.mark.parametrize("theta", [[1.0, 0, 0, 0], [1.0, 0.3, -0.2, 0.5]])
+def test_f16_solves_with_phases(L, theta):
+    conf = conf_of(L, 52, theta)
+    geo = orc.Geom(L)
+    kappa, mus, n = 0.16, [0.05, 0.07, 0.09], 3
+    src = [nq.source_lx(L, 70 + i) for i in range(n)]
+    ref = [geo.tm_solve_eoprec(conf, kappa, mus[i], 20000, 1e-24, src[i])[0] for i in range(n)]
+    ce, co = geo.split(conf)
+    x = gauss_eo(geo.Vh, 8)
+    with nq.Ctx(L) as ctx:
+        g = nq.Gauge(ctx, lx=conf)
+        fi, fo = ctx.field(nq.SPINCOLOR, nq.ODD, x), ctx.field(nq.SPINCOLOR, nq.EVEN)
+        nq.tm_hop(ctx, g, fo, fi)
+        assert rel_l2(fo.download(), geo.tm_hop(0, ce, co, x)) < 1e-14
+        fs = [ctx.field(nq.SPINCOLOR, nq.LX, s) for s in src]
+        fx = [ctx.field(nq.SPINCOLOR, nq.LX) for _ in src]
+        for prec in ("f16", "f16h", "f32"):
+            st = nq.tm_solve_eoprec(ctx, g, kappa, mus[0], 20000, 1e-24, fx[0], fs[0], prec=prec)
+            assert st["rc"] == nq.NQ_OK
+            assert rel_l2(fx[0].download(), ref[0]) < 1e-10, prec
+            res = nq.tm_solve_eoprec_multi(ctx, g, kappa, mus, 20000, 1e-24, fx, fs, prec=prec)
+            assert all(r["rc"] == nq.NQ_OK for r in res)
+            for i in range(n):
+                assert rel_l2(fx[i].download(), ref[i]) < 1e-10, (prec, i)
