@@ -192,34 +192,6 @@ __global__ void __launch_bounds__(256) k_pupdate_pair(BlasArgs A, SpinorView pin
   store_any<NC>(pout, A.g.stride, m.e, pv, m.r);
 }
 
-// x += alpha p ; r -= alpha s ; |r|^2 (plain CG update, cg_invert_template_threaded.hpp:82-102)
-template <int NC>
-__global__ void __launch_bounds__(256) k_cg_update(BlasArgs A, SpinorView x, SpinorView p, SpinorView r, SpinorView s)
-{
-  const Map m = map_thread(A.s, A.g.Vh);
-  const CgState* S = A.st + m.r;
-  double nrm = 0;
-  if (m.active && !S->done && !S->reliable) {
-    const double alpha = S->alpha;
-    cx<double> xv[NC], pv[NC], rv[NC], sv[NC];
-    load_any<NC>(x, A.g.stride, m.e, xv, m.r);
-    load_any<NC>(p, A.g.stride, m.e, pv, m.r);
-    load_any<NC>(r, A.g.stride, m.e, rv, m.r);
-    load_any<NC>(s, A.g.stride, m.e, sv, m.r);
-#pragma unroll
-    for (int k = 0; k < NC; k++) {
-      xv[k].re = fma(alpha, pv[k].re, xv[k].re);
-      xv[k].im = fma(alpha, pv[k].im, xv[k].im);
-      rv[k].re = fma(-alpha, sv[k].re, rv[k].re);
-      rv[k].im = fma(-alpha, sv[k].im, rv[k].im);
-      nrm += rv[k].re * rv[k].re + rv[k].im * rv[k].im;
-    }
-    store_any<NC>(x, A.g.stride, m.e, xv, m.r);
-    store_any<NC>(r, A.g.stride, m.e, rv, m.r);
-  }
-  store_partial(nrm, A.partial, A.nchunks, m.r, m.chunk);
-}
-
 // x64 += xs ; xs = 0 (reliable update), only for right-hand sides flagged reliable
 template <int NC>
 __global__ void __launch_bounds__(256) k_reliable_accum(BlasArgs A, SpinorView x64, SpinorView xs, SpinorView p,
@@ -307,10 +279,10 @@ __global__ void __launch_bounds__(1024) k_finalize(const double* partial, int64_
   if (threadIdx.x == 0) finalize(s, fin, tot);
 }
 
-int launch_finalize(nq_ctx* ctx, int nr, CgState* st, int fin, int pred_reliable)
+int launch_finalize(nq_ctx* ctx, int nr, CgState* st, int fin, int pred_reliable, int64_t nchunks)
 {
   if (!st || fin == FIN_NONE) return fail(NQ_EINVAL, "finalize without state");
-  const int64_t nchunks = (ctx->geo.Vh + 63) / 64;
+  if (nchunks <= 0) nchunks = (ctx->geo.Vh + 63) / 64;
   hipEvent_t ev = nullptr;
   prof_begin(ctx, "reduce_finalize", 8.0 * nchunks * nr, &ev);
   hipLaunchKernelGGL(k_finalize, dim3(nr), dim3(1024), 0, ctx->stream, ctx->partial, nchunks, st, fin, pred_reliable);
@@ -448,24 +420,6 @@ int launch_cg_pupdate(nq_ctx* ctx, const SpinorView& p, const SpinorView& r, CgS
   NQ_HIP(hipGetLastError());
   prof_end(ctx, ev);
   return NQ_OK;
-}
-
-int launch_cg_update(nq_ctx* ctx, const SpinorView& x, const SpinorView& p, const SpinorView& r, const SpinorView& s,
-                     CgState* st, int fin, int nr)
-{
-  BlasArgs A;
-  Launch L;
-  NQ_TRY(make_args(ctx, nr, st, fin, 1, &A, &L));
-  hipEvent_t ev = nullptr;
-  prof_begin(ctx, "blas_cg_update",
-             nr * (2 * site_bytes(x) + site_bytes(p) + 2 * site_bytes(r) + site_bytes(s)) * (double)ctx->geo.Vh, &ev);
-  const dim3 grid((unsigned)L.blocks), blk(L.threads);
-  if (x.ncomp == 24) hipLaunchKernelGGL(k_cg_update<24>, grid, blk, 0, ctx->stream, A, x, p, r, s);
-  else if (x.ncomp == 12) hipLaunchKernelGGL(k_cg_update<12>, grid, blk, 0, ctx->stream, A, x, p, r, s);
-  else hipLaunchKernelGGL(k_cg_update<3>, grid, blk, 0, ctx->stream, A, x, p, r, s);
-  NQ_HIP(hipGetLastError());
-  prof_end(ctx, ev);
-  return launch_finalize(ctx, nr, st, fin, 2);
 }
 
 __global__ void k_clear_reliable(CgState* st, int nr)

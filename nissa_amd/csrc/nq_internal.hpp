@@ -126,6 +126,14 @@ struct CgmState {
   int owe[kMaxShift];
   int done, reliable;  // adjacent: the sloppy kernels skip a source when either is set
   int nshift, nrun, iter, niter, nan, mixed, kref, nreliable;
+  // lx solves (launch_cgm_vec): the shift vectors are updated every other iteration, from
+  // the pending iteration's coefficients (b1, z1, a1; ran1: shifts that ran in it; ran2:
+  // in the current one).  vmode, set by the rfrf finalisation, is the next vector
+  // update's work: 0 none (idle after the end), 1 p only, keeping r (this iteration stays
+  // pending), 2 p and both iterations, 3 the last iteration alone (the end came on one)
+  double b1[kMaxShift], z1[kMaxShift], a1[kMaxShift];
+  int ran1[kMaxShift], ran2[kMaxShift];
+  int lx, vlag, vmode, pad1;
   // pend: the ps_k update of the iteration just finalised is left to the next
   // iteration's hop2 kernel (set by the rfrf finalisation when the source goes on
   // without a reliable update; the update kernel then updates p only)
@@ -173,6 +181,9 @@ struct HopEpi {
   // other kernels launch it separately): fold_fin on st with predicate fold_pred
   int fold_fin = FIN_NONE;
   int fold_pred = 0;
+  // chunk partials of a reduction go to the context's scratch from this index on (FIN_PARTIAL:
+  // the lx solvers reduce both parities in one finalisation)
+  int64_t part0 = 0;
   // twisted clover blocks in the epilogue (clover_block.hpp): blk_mode 1 applies the
   // inverse blocks blk (72 complex per site) to the hop before c1; blk_mode 2 applies
   // the blocks z + clover term (blk: 36 complex per site, z = 1/(2 blk_kappa) +- i
@@ -333,15 +344,14 @@ int launch_st_hop(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& 
 // reliable update when only_reliable)
 int launch_cgm_flush(nq_ctx* ctx, const SpinorView& sol64, const SpinorView& sol, int64_t sstride, int nshift,
                      void* states, int nr, int only_reliable);
-// generic multi-shift CG pieces for lx spincolor fields (one source, FP64):
-// finalisation of the reduction just launched (fin 1: <p,A p> = pap_scale * sum,
-// 2: |r|^2), v2: sol_k -= betas_k ps_k, r += betaa s, |r|^2 (+ finalisation),
-// v3: p = r + alpha p, ps_k = zfs_k r + alphas_k ps_k
-int launch_cgm_finalize(nq_ctx* ctx, void* states, int nr, int fin, double pap_scale);
-int launch_cgm_vec2(nq_ctx* ctx, const SpinorView& s, const SpinorView& r, const SpinorView& sol, const SpinorView& ps,
-                    int64_t sstride, void* states);
-int launch_cgm_vec3(nq_ctx* ctx, const SpinorView& r, const SpinorView& p, const SpinorView& ps, int64_t sstride,
-                    void* states);
+// multi-shift CG pieces for lx spincolor fields (one source, FP64): finalisation of the
+// reduction just launched over both parities' chunks (fin 1: <p,A p> = sum, 2: |r|^2),
+// which also sets mirror->alpha (-betaa) and mirror->done for the hop epilogues; and the
+// vector update p = r + alpha p, sol_k -= betas_k ps_k, ps_k = zfs_k r + alphas_k ps_k
+// (the shifts every other iteration, rprev holding the pending iteration's r)
+int launch_cgm_finalize_lx(nq_ctx* ctx, void* states, int fin, CgState* mirror);
+int launch_cgm_vec(nq_ctx* ctx, const SpinorView& r, const SpinorView& rprev, const SpinorView& p,
+                   const SpinorView& sol, const SpinorView& ps, int64_t sstride, void* states, int nshift);
 // one multi-shift CG iteration for nr sources (states: device CgmState[nr]);
 // sol/ps hold the shifts of each source at element offset k*sstride; nbusy and nrun
 // (sources still iterating and their running shifts, as the host last saw them) only
@@ -415,10 +425,6 @@ int launch_cg_pupdate(nq_ctx* ctx, const SpinorView& p, const SpinorView& r, CgS
                       const SpinorView& x = SpinorView());
 // state[i].reliable = 0 for i < nr
 int launch_clear_reliable(nq_ctx* ctx, CgState* st, int nr);
-// x += alpha p ; r -= alpha s ; |r|^2 -> fin  (alpha from state, skipped when done or
-// while a reliable update is due)
-int launch_cg_update(nq_ctx* ctx, const SpinorView& x, const SpinorView& p, const SpinorView& r,
-                     const SpinorView& s, CgState* st, int fin, int nr = 1);
 int launch_reliable_accum(nq_ctx* ctx, const SpinorView& x64, const SpinorView& xs, CgState* st, int nr = 1,
                           const SpinorView& p = SpinorView(), const SpinorView& p_prev = SpinorView());
 // p_out = r + beta p_in (one right-hand side, p_in and p_out distinct; skipped when done or
@@ -435,6 +441,7 @@ int launch_spin_diag(nq_ctx* ctx, const SpinorView& out, const double a[2][2], c
 int reduce_norm2(nq_ctx* ctx, const SpinorView& v, double* out);
 // sum the per-chunk partials of the last reducing launch into state[0..nr) with fin;
 // pred_reliable as in HopEpi (the same condition the reducing launch used)
-int launch_finalize(nq_ctx* ctx, int nr, CgState* st, int fin, int pred_reliable);
+// nchunks: number of partials per right-hand side (0: one parity's chunks)
+int launch_finalize(nq_ctx* ctx, int nr, CgState* st, int fin, int pred_reliable, int64_t nchunks = 0);
 int reduce_dot(nq_ctx* ctx, const SpinorView& a, const SpinorView& b, double* out);
 }  // namespace nq

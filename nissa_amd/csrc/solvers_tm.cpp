@@ -434,10 +434,20 @@ static int cg_kernsq_any(nq_ctx* ctx, const nq_gauge* g, double kappa, const dou
   return cg_kernsq_mixed(S64, Ss, sp, mu, niter, residue, reliable_delta(sp, residue), x, guess, b, st, kx);
 }
 
+// Q(mu) on parity p of lx fields; `last` carries the epilogue's mode and tail, whose
+// c1, c2 and aux are set here
+static int apply_Q_parity(const TmSetup& S, double mu, int p, const SpinorView& out, const nq_field* in, HopEpi last)
+{
+  const HopEpi e = epi_q(S.kappa, mu, view_of(in, p));
+  std::memcpy(last.c1, e.c1, sizeof e.c1);
+  std::memcpy(last.c2, e.c2, sizeof e.c2);
+  last.aux = e.aux;
+  return launch_tm_hop(S.ctx, p, out, view_of(in, !p), S.U, S.anis, last);
+}
+
 static int apply_Q_views(const TmSetup& S, double mu, const nq_field* out, const nq_field* in)
 {
-  for (int p = 0; p < 2; p++)
-    NQ_TRY(launch_tm_hop(S.ctx, p, view_of(out, p), view_of(in, !p), S.U, S.anis, epi_q(S.kappa, mu, view_of(in, p))));
+  for (int p = 0; p < 2; p++) NQ_TRY(apply_Q_parity(S, mu, p, view_of(out, p), in, HopEpi()));
   return NQ_OK;
 }
 
@@ -1151,8 +1161,50 @@ int TmBatch::finish(int slot, const SpinorView& src_e, const SpinorView& src_o, 
 }
 
 // CG on Q(-mu) Q(+mu) over lx (inv_tmQ2_cg), FP64, cg_invert semantics
-// Q(mu) on lx fields: writes out = Q(mu) in
-typedef std::function<int(double mu, const nq_field* out, const nq_field* in)> ApplyQ;
+// Q(mu) on lx fields, one parity of the output at a time: the hop of parity p with the
+// epilogue mode and tail of `last`
+typedef std::function<int(double mu, int p, const SpinorView& out, const nq_field* in, const HopEpi& last)> ApplyQ;
+
+static int apply_q(const ApplyQ& Q, double mu, const nq_field* out, const nq_field* in)
+{
+  for (int p = 0; p < 2; p++) NQ_TRY(Q(mu, p, view_of(out, p), in, HopEpi()));
+  return NQ_OK;
+}
+
+// The two halves of s = Q(-mu) Q(+mu) p inside an lx CG, with the reductions and the
+// r update (and x += alpha p, when x is given) in the hop epilogues, each parity's chunk
+// partials after the other's: t = Q(+mu) p with |t|^2, then r -= alpha Q(-mu) t with
+// |r|^2.  s is never stored, and no pass of its own forms a norm.
+static int q2_first(nq_ctx* ctx, const ApplyQ& Q, double mu, const nq_field* t, const nq_field* p, CgState* st)
+{
+  for (int par = 0; par < 2; par++) {
+    HopEpi e;
+    e.mode = 1;
+    e.st = st;
+    e.fin = FIN_PARTIAL;
+    e.part0 = par * ((ctx->geo.Vh + 63) / 64);
+    NQ_TRY(Q(mu, par, view_of(t, par), p, e));
+  }
+  return NQ_OK;
+}
+static int q2_second(nq_ctx* ctx, const ApplyQ& Q, double mu, const nq_field* t, const nq_field* r, const nq_field* p,
+                     const nq_field* x, CgState* st)
+{
+  SpinorView none;
+  none.ncomp = 12;
+  for (int par = 0; par < 2; par++) {
+    HopEpi e;
+    e.mode = 2;
+    e.st = st;
+    e.fin = FIN_PARTIAL;
+    e.part0 = par * ((ctx->geo.Vh + 63) / 64);
+    e.r = view_of(r, par);
+    e.p = view_of(p, par);
+    if (x) e.x = view_of(x, par);
+    NQ_TRY(Q(-mu, par, none, t, e));
+  }
+  return NQ_OK;
+}
 
 // cg_invert on Q(-mu)Q(+mu) over lx fields (inv_tmQ2_cg / inv_tmclovQ2_cg): the matvec
 // is two Q applies and <p, Q(-mu)Q(+mu) p> = |Q(+mu) p|^2 (Q(mu)^+ = Q(-mu)).  FP64.
@@ -1198,8 +1250,8 @@ static int q2_cg_f64(nq_ctx* ctx, const ApplyQ& Q, double mu, int niter, double 
   s0.niter = niter;
   NQ_TRY(put_state(ctx, 0, s0));
   auto q2 = [&](const nq_field* out_f, const nq_field* in_f) -> int {
-    NQ_TRY(Q(+mu, &ft, in_f));
-    return Q(-mu, out_f, &ft);
+    NQ_TRY(apply_q(Q, +mu, &ft, in_f));
+    return apply_q(Q, -mu, out_f, &ft);
   };
   if (guess) {
     if (guess != sol) NQ_TRY(launch_convert(ctx, x, view_lx_flat(guess)));
@@ -1215,11 +1267,12 @@ static int q2_cg_f64(nq_ctx* ctx, const ApplyQ& Q, double mu, int niter, double 
   int chunk = 8, launched = 0;
   while (!ctx->state_host[0].done) {
     for (int i = 0; i < chunk; i++) {
-      // s = Q(-mu) Q(+mu) p ; <p, s> = |Q(+mu) p|^2
-      NQ_TRY(Q(+mu, &ft, &fp));
-      NQ_TRY(launch_lincomb(ctx, none, 1.0, view_lx_flat(&ft), 0, none, 0, none, FIN_PAP, st, 1, 1));
-      NQ_TRY(Q(-mu, &fs, &ft));
-      NQ_TRY(launch_cg_update(ctx, x, p, r, s, st, FIN_RR));
+      // s = Q(-mu) Q(+mu) p ; <p, s> = |Q(+mu) p|^2 ; x += alpha p ; r -= alpha s
+      const int64_t nparts = 2 * ((ctx->geo.Vh + 63) / 64);
+      NQ_TRY(q2_first(ctx, Q, mu, &ft, &fp, st));
+      NQ_TRY(launch_finalize(ctx, 1, st, FIN_PAP, 0, nparts));
+      NQ_TRY(q2_second(ctx, Q, mu, &ft, &fr, &fp, sol, st));
+      NQ_TRY(launch_finalize(ctx, 1, st, FIN_RR, 0, nparts));
       NQ_TRY(launch_cg_pupdate(ctx, p, r, st));
     }
     launched += chunk;
@@ -1252,7 +1305,8 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
                       double* true_res)
 {
   const int64_t fsz = 24 * ctx->geo.stride;  // elements of one lx field
-  SpinorView rv, pv, tv, sv, ps, xs;
+  SpinorView rv, pv, tv, sv, qv, ps, xs;
+  NQ_TRY(alloc_spinor_nr(ctx, "q2m.rprev", SP_F64, 24, 1, &qv));
   NQ_TRY(alloc_spinor_nr(ctx, "q2.r", SP_F64, 12, 2, &rv));
   NQ_TRY(alloc_spinor_nr(ctx, "q2.p", SP_F64, 12, 2, &pv));
   NQ_TRY(alloc_spinor_nr(ctx, "q2.t", SP_F64, 12, 2, &tv));
@@ -1275,8 +1329,7 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
       for (auto* x : f) x->buf.p = nullptr;
     }
   } rel{{&fr, &fp, &ft, &fs}};
-  const SpinorView b = view_lx_flat(src), r = view_lx_flat(&fr), p = view_lx_flat(&fp), t = view_lx_flat(&ft),
-                   s = view_lx_flat(&fs);
+  const SpinorView b = view_lx_flat(src), r = view_lx_flat(&fr), p = view_lx_flat(&fp), s = view_lx_flat(&fs);
   SpinorView none;
   none.ncomp = 24;
   Timer T(ctx->stream);
@@ -1300,6 +1353,7 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
   h0.nshift = nmass;
   h0.nrun = nmass;
   h0.niter = niter;
+  h0.lx = 1;
   for (int k = 0; k < nmass; k++) {
     h0.shift[k] = masses[k] * masses[k];
     h0.target[k] = residues[k];
@@ -1317,22 +1371,27 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
   }
   NQ_TRY(launch_convert(ctx, p, b));
   NQ_TRY(launch_convert(ctx, r, b));
-  int chunk = 8, launched = 0;
+  // alpha (-betaa) and the stop flag of the source, for the hop epilogues
+  NQ_TRY(put_state(ctx, 0, CgState{}));
+  CgState* mirror = ctx->state;
+  int chunk = 8, launched = 0, kref = 0;
+  for (int k = 1; k < nmass; k++)
+    if (masses[k] * masses[k] < masses[kref] * masses[kref]) kref = k;
   for (;;) {
     for (int it = 0; it < chunk; it++) {
-      NQ_TRY(Q(0.0, &ft, &fp));  // t = Q(0) p
-      NQ_TRY(launch_lincomb(ctx, none, 1.0, t, 0, none, 0, none, FIN_PARTIAL, nullptr));
-      NQ_TRY(launch_cgm_finalize(ctx, dst, 1, 1, 1.0));  // pap = |t|^2
-      NQ_TRY(Q(0.0, &fs, &ft));  // s = Q(0)^2 p
-      NQ_TRY(launch_cgm_vec2(ctx, s, r, xs, ps, fsz, dst));
-      NQ_TRY(launch_cgm_vec3(ctx, r, p, ps, fsz, dst));
+      NQ_TRY(q2_first(ctx, Q, 0.0, &ft, &fp, mirror));  // t = Q(0) p, |t|^2
+      NQ_TRY(launch_cgm_finalize_lx(ctx, dst, 1, mirror));  // pap = |t|^2
+      NQ_TRY(q2_second(ctx, Q, 0.0, &ft, &fr, &fp, nullptr, mirror));  // r += betaa Q(0) t, |r|^2
+      NQ_TRY(launch_cgm_finalize_lx(ctx, dst, 2, mirror));
+      NQ_TRY(launch_cgm_vec(ctx, r, qv, p, xs, ps, fsz, dst, nmass));
     }
     launched += chunk;
     NQ_HIP(hipMemcpyAsync(hst, dst, sizeof(CgmState), hipMemcpyDeviceToHost, ctx->stream));
     NQ_HIP(hipStreamSynchronize(ctx->stream));
     if (hst->nan) return fail(NQ_ENAN, "nanned");
     if (hst->done || launched > niter + 64) break;
-    chunk = std::min(64, chunk * 2);
+    // the shift of the smallest mass converges last
+    chunk = next_chunk(1.0, hst->res[kref], residues[kref], hst->iter, std::min(64, chunk * 2));
   }
   const int iters = hst->iter;
   // copy out and the FP64 check |(Q(-m)Q(+m)) x_k - b|^2 / |b|^2
@@ -1341,8 +1400,8 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
     SpinorView xk = xs;
     xk.data = (char*)xs.data + k * fsz * 16;
     NQ_TRY(launch_convert(ctx, view_lx_flat(sols[k]), xk));
-    NQ_TRY(Q(+masses[k], &ft, sols[k]));
-    NQ_TRY(Q(-masses[k], &fs, &ft));
+    NQ_TRY(apply_q(Q, +masses[k], &ft, sols[k]));
+    NQ_TRY(apply_q(Q, -masses[k], &fs, &ft));
     NQ_TRY(put_state(ctx, 0, CgState{}));
     NQ_TRY(launch_lincomb(ctx, none, 1.0, s, -1.0, b, 0, none, FIN_STORE0, ctx->state));
     NQ_TRY(get_states(ctx, 0, 1));
@@ -1729,7 +1788,9 @@ int nq_tmQ2_cg(nq_ctx* c, const nq_gauge* g, double kappa, double mu, int niter,
   nq_solve_stats local;
   if (!st) st = &local;
   std::memset(st, 0, sizeof *st);
-  const ApplyQ Q = [&](double m, const nq_field* o, const nq_field* i) { return apply_Q_views(S, m, o, i); };
+  const ApplyQ Q = [&](double m, int par, const SpinorView& o, const nq_field* i, const HopEpi& e) {
+    return apply_Q_parity(S, m, par, o, i, e);
+  };
   return q2_cg_f64(c, Q, mu, niter, residue, sol, guess, src, st);
 }
 
@@ -1761,7 +1822,9 @@ int nq_tmQ2_cgm(nq_ctx* c, const nq_gauge* g, double kappa, int nmass, const dou
   Guard G(c);
   TmSetup S;
   NQ_TRY(tm_setup(c, g, LK_F64_18, nullptr, kappa, &S));
-  const ApplyQ Q = [&](double m, const nq_field* o, const nq_field* i) { return apply_Q_views(S, m, o, i); };
+  const ApplyQ Q = [&](double m, int par, const SpinorView& o, const nq_field* i, const HopEpi& e) {
+    return apply_Q_parity(S, m, par, o, i, e);
+  };
   return q2_cgm_f64(c, Q, nmass, masses, niter, residues, sols, src, st, true_res);
 }
 
@@ -2220,19 +2283,22 @@ int nq_tmclov_kern_square(nq_ctx* c, const nq_gauge* g, nq_clover* cl, double ka
 
 // Q = g5 D, D = 1/(2 kappa) + i mu g5 + Cl - 1/2 hop on each parity
 // apply_tmclovQ on lx views: per parity, out = gamma5 (D_pp-block in_p - 1/2 hop in_!p)
-static int clov_apply_Q_views(const TmSetup& S, nq_clover* cl, double mu, const nq_field* out, const nq_field* in)
+static int clov_apply_Q_parity(const TmSetup& S, nq_clover* cl, double mu, int p, const SpinorView& out,
+                               const nq_field* in, HopEpi last)
 {
   nq_ctx* c = S.ctx;
   SpinorView u, none;
   NQ_TRY(alloc_spinor(c, "clov.uo", SP_F64, 12, &u));
-  for (int p = 0; p < 2; p++) {
-    NQ_TRY(launch_clover_apply(c, 0, u, view_of(in, p), clov_view(cl, p), none, S.kappa, mu, 0, kOne, nullptr));
-    HopEpi e;
-    setc(e.c1, -0.5, 0.5);
-    setc(e.c2, 1.0, -1.0);
-    e.aux = u;
-    NQ_TRY(launch_tm_hop(c, p, view_of(out, p), view_of(in, !p), S.U, S.anis, e));
-  }
+  NQ_TRY(launch_clover_apply(c, 0, u, view_of(in, p), clov_view(cl, p), none, S.kappa, mu, 0, kOne, nullptr));
+  setc(last.c1, -0.5, 0.5);
+  setc(last.c2, 1.0, -1.0);
+  last.aux = u;
+  return launch_tm_hop(c, p, out, view_of(in, !p), S.U, S.anis, last);
+}
+
+static int clov_apply_Q_views(const TmSetup& S, nq_clover* cl, double mu, const nq_field* out, const nq_field* in)
+{
+  for (int p = 0; p < 2; p++) NQ_TRY(clov_apply_Q_parity(S, cl, mu, p, view_of(out, p), in, HopEpi()));
   return NQ_OK;
 }
 
@@ -2301,7 +2367,9 @@ int nq_tmclovQ2_cg(nq_ctx* c, const nq_gauge* g, nq_clover* cl, double kappa, co
   nq_solve_stats local;
   if (!st) st = &local;
   std::memset(st, 0, sizeof *st);
-  const ApplyQ Q = [&](double m, const nq_field* o, const nq_field* i) { return clov_apply_Q_views(S, cl, m, o, i); };
+  const ApplyQ Q = [&](double m, int par, const SpinorView& o, const nq_field* i, const HopEpi& e) {
+    return clov_apply_Q_parity(S, cl, m, par, o, i, e);
+  };
   return q2_cg_f64(c, Q, mu, niter, residue, sol, guess, src, st);
 }
 
@@ -2323,7 +2391,9 @@ int nq_tmclovQ2_cgm(nq_ctx* c, const nq_gauge* g, nq_clover* cl, double kappa, c
   Guard G(c);
   TmSetup S;
   NQ_TRY(tm_setup(c, g, LK_F64_18, anis, kappa, &S));
-  const ApplyQ Q = [&](double m, const nq_field* o, const nq_field* i) { return clov_apply_Q_views(S, cl, m, o, i); };
+  const ApplyQ Q = [&](double m, int par, const SpinorView& o, const nq_field* i, const HopEpi& e) {
+    return clov_apply_Q_parity(S, cl, m, par, o, i, e);
+  };
   return q2_cgm_f64(c, Q, nmass, masses, niter, residues, sols, src, st, true_res);
 }
 

@@ -532,6 +532,16 @@ __device__ inline void cgm_finalize(CgmState* s, int fin, double total, double p
       s->zps[k] = s->zas[k];
       s->zas[k] = s->zfs[k];
     }
+    if (s->lx)
+      for (int k = 0; k < s->nshift; k++) {
+        if (!s->vlag) {  // this iteration may stay pending
+          s->b1[k] = s->betas[k];
+          s->z1[k] = s->zfs[k];
+          s->a1[k] = s->alphas[k];
+          s->ran1[k] = s->run[k];
+        }
+        s->ran2[k] = s->run[k];
+      }
     s->rr = rfrf;
     s->iter += 1;
     // the C2 just run left its sol_k terms when lag was clear (the next C2 applies
@@ -567,6 +577,12 @@ __device__ inline void cgm_finalize(CgmState* s, int fin, double total, double p
     // reliable update (which replaces r) comes first
     s->pend = !s->done && !s->reliable;
     s->lag = owed && s->pend;
+    if (s->lx) {
+      // the vector update of this iteration (CgmState::vmode)
+      if (s->vlag) s->vmode = 2;
+      else s->vmode = s->done ? 3 : 1;
+      s->vlag = s->vmode == 1;
+    }
   }
 }
 
@@ -940,116 +956,92 @@ int launch_cgm_flush(nq_ctx* ctx, const SpinorView& x64, const SpinorView& sol, 
   return NQ_OK;
 }
 
-// ------------------------------------------------------------------ generic CGM vectors
-// For operators whose matvec is launched separately (the lx twisted-mass Q^2):
-//   v2: sol_k -= betas_k ps_k (running k) ; r += betaa s ; |r|^2
-//   v3: p = r + alpha p ; ps_k = zfs_k r + alphas_k ps_k (running k)
-// FP64 fields of NC complex components; one source (state st[0]).
-template <int NC>
-__global__ void __launch_bounds__(256) k_cgm_vec2(Geo g, SpinorView s, SpinorView r, SpinorView sol, SpinorView ps,
-                                                  int64_t sstride, const CgmState* st, Shape SH, int64_t nchunks,
-                                                  double* partial)
+// ------------------------------------------------------------------ lx CGM vectors
+// Multi-shift CG on Q^2 over lx fields (the matvec and the r update are hop epilogues):
+// p = r + alpha p, and for the shifts sol_k -= betas_k ps_k ; ps_k = zfs_k r + alphas_k ps_k.
+// The shifts are visited every other iteration (CgmState::vmode), two iterations at a
+// time and in order, so ps_k and sol_k move half as often; the bits are those of one
+// update per iteration.  Bound by bandwidth (the fields of a 16^3x32 lattice sit in the
+// memory-side cache): one 16-byte element a thread, so that a small lattice still fills
+// the chip.  Two separate kernels that wrote and re-read s and visited the shifts every
+// iteration took 52 + 39 us an iteration with four shifts at 16^3x32.
+__global__ void __launch_bounds__(256) k_cgm_vec(int64_t n, const double2* __restrict__ r, double2* __restrict__ rprev,
+                                                 double2* __restrict__ p, double2* __restrict__ sol,
+                                                 double2* __restrict__ ps, int64_t sstride, const CgmState* st)
 {
-  const Map m = map_thread(SH, g.Vh);
-  double red = 0;
-  if (m.active && !st->done) {
-    for (int k = 0; k < st->nshift; k++) {
-      if (!st->run[k]) continue;
-      SpinorView sk = sol, pk = ps;
-      sk.data = (char*)sol.data + k * sstride * 16;
-      pk.data = (char*)ps.data + k * sstride * 16;
-      cx<double> x[NC], q[NC];
-      SpAcc<SP_F64, double, NC, kNT>::load(sk, g.stride, m.e, x);
-      SpAcc<SP_F64, double, NC, kNT>::load(pk, g.stride, m.e, q);
-      const double b = st->betas[k];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        x[c].re = fma(-b, q[c].re, x[c].re);
-        x[c].im = fma(-b, q[c].im, x[c].im);
-      }
-      SpAcc<SP_F64, double, NC, kNT>::store(sk, g.stride, m.e, x);
-    }
-    cx<double> rv[NC], sv[NC];
-    SpAcc<SP_F64, double, NC>::load(r, g.stride, m.e, rv);
-    SpAcc<SP_F64, double, NC, kNT>::load(s, g.stride, m.e, sv);
-    const double ba = st->betaa;
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      rv[c].re = fma(ba, sv[c].re, rv[c].re);
-      rv[c].im = fma(ba, sv[c].im, rv[c].im);
-      red += rv[c].re * rv[c].re + rv[c].im * rv[c].im;
-    }
-    SpAcc<SP_F64, double, NC>::store(r, g.stride, m.e, rv);
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int mode = sload(&st->vmode);
+  if (mode == 0 || i >= n) return;
+  auto axpy = [](double a, double2 x, double2 y) { return make_double2(fma(a, x.x, y.x), fma(a, x.y, y.y)); };
+  auto scale = [](double a, double2 x) { return make_double2(a * x.x, a * x.y); };
+  const double2 rv = r[i];
+  const bool done = sload(&st->done) != 0;
+  if (!done) p[i] = axpy(sload(&st->alpha), p[i], rv);
+  if (mode == 1) {
+    rprev[i] = rv;
+    return;
   }
-  store_partial(red, partial, nchunks, 0, m.chunk);
-}
-
-template <int NC>
-__global__ void __launch_bounds__(256) k_cgm_vec3(Geo g, SpinorView r, SpinorView p, SpinorView ps, int64_t sstride,
-                                                  const CgmState* st, Shape SH)
-{
-  const Map m = map_thread(SH, g.Vh);
-  if (!m.active || st->done) return;
-  cx<double> rv[NC], pv[NC];
-  SpAcc<SP_F64, double, NC>::load(r, g.stride, m.e, rv);
-  SpAcc<SP_F64, double, NC>::load(p, g.stride, m.e, pv);
-  const double a = st->alpha;
-#pragma unroll
-  for (int c = 0; c < NC; c++) {
-    pv[c].re = fma(a, pv[c].re, rv[c].re);
-    pv[c].im = fma(a, pv[c].im, rv[c].im);
-  }
-  SpAcc<SP_F64, double, NC>::store(p, g.stride, m.e, pv);
-  for (int k = 0; k < st->nshift; k++) {
-    if (!st->run[k]) continue;
-    SpinorView pk = ps;
-    pk.data = (char*)ps.data + k * sstride * 16;
-    cx<double> q[NC];
-    SpAcc<SP_F64, double, NC, kNT>::load(pk, g.stride, m.e, q);
-    const double z = st->zfs[k], al = st->alphas[k];
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      q[c].re = fma(al, q[c].re, z * rv[c].re);
-      q[c].im = fma(al, q[c].im, z * rv[c].im);
+  const double2 r1 = mode == 2 ? rprev[i] : rv;
+  const int ns = sload(&st->nshift);
+  for (int k = 0; k < ns; k++) {
+    const bool ran2 = sload(&st->ran2[k]) != 0, ran1 = mode == 2 && sload(&st->ran1[k]) != 0;
+    if (!ran1 && !ran2) continue;  // uniform over the launch
+    double2 q = ps[k * sstride + i], x = sol[k * sstride + i];
+    if (ran1) {
+      x = axpy(-sload(&st->b1[k]), q, x);
+      q = axpy(sload(&st->a1[k]), q, scale(sload(&st->z1[k]), r1));
     }
-    SpAcc<SP_F64, double, NC, kNT>::store(pk, g.stride, m.e, q);
+    if (ran2) {
+      x = axpy(-sload(&st->betas[k]), q, x);
+      if (!done && sload(&st->run[k])) ps[k * sstride + i] = axpy(sload(&st->alphas[k]), q, scale(sload(&st->zfs[k]), rv));
+    }
+    sol[k * sstride + i] = x;
   }
 }
 
-int launch_cgm_finalize(nq_ctx* ctx, void* states, int nr, int fin, double pap_scale)
+// k_cgm_finalize over nparts partials of one source, which also hands alpha and the stop
+// flag to the hop epilogues and clears the vector update's work once the source is done
+__global__ void __launch_bounds__(1024) k_cgm_finalize_lx(const double* partial, int64_t nparts, CgmState* s, int fin,
+                                                          CgState* mirror)
 {
-  const int64_t nchunks = (ctx->geo.Vh + 63) / 64;
-  hipLaunchKernelGGL(k_cgm_finalize, dim3(nr), dim3(1024), 0, ctx->stream, ctx->partial, nchunks, (CgmState*)states,
-                     fin == 1 ? (int)FIN_CGM_PAP : (int)FIN_CGM_RFRF, pap_scale);
+  __shared__ double vl[1024];
+  if (s->done) {  // uniform over the workgroup
+    if (threadIdx.x == 0) s->vmode = 0;
+    return;
+  }
+  const double tot = block_sum_partials(partial, nparts, vl);
+  if (threadIdx.x == 0) {
+    cgm_finalize(s, fin, tot, 1.0);
+    mirror->alpha = -s->betaa;
+    mirror->done = s->done;
+  }
+}
+
+int launch_cgm_finalize_lx(nq_ctx* ctx, void* states, int fin, CgState* mirror)
+{
+  const int64_t nparts = 2 * ((ctx->geo.Vh + 63) / 64);
+  hipEvent_t ev = nullptr;
+  prof_begin(ctx, "reduce_finalize", 8.0 * nparts, &ev);
+  hipLaunchKernelGGL(k_cgm_finalize_lx, dim3(1), dim3(1024), 0, ctx->stream, ctx->partial, nparts, (CgmState*)states,
+                     fin == 1 ? (int)FIN_CGM_PAP : (int)FIN_CGM_RFRF, mirror);
   NQ_HIP(hipGetLastError());
+  prof_end(ctx, ev);
   return NQ_OK;
 }
 
-int launch_cgm_vec2(nq_ctx* ctx, const SpinorView& s, const SpinorView& r, const SpinorView& sol, const SpinorView& ps,
-                    int64_t sstride, void* states)
+int launch_cgm_vec(nq_ctx* ctx, const SpinorView& r, const SpinorView& rprev, const SpinorView& p,
+                   const SpinorView& sol, const SpinorView& ps, int64_t sstride, void* states, int nshift)
 {
-  const Geo& g = ctx->geo;
-  const Launch L = launch_shape(g, 1);
-  if (r.ncomp != 24) return fail(NQ_EINVAL, "cgm vectors: lx spincolor fields expected");
+  if (r.ncomp != 24 || p.ncomp != 24 || rprev.ncomp != 24 || r.prec != SP_F64)
+    return fail(NQ_EINVAL, "cgm vectors: FP64 lx spincolor fields expected");
+  const int64_t n = 24 * ctx->geo.stride;
+  if (sstride < n) return fail(NQ_EINVAL, "cgm vectors: shift stride below one field");
   hipEvent_t ev = nullptr;
-  prof_begin(ctx, "cgm_vec2", 0.0, &ev);
-  hipLaunchKernelGGL(k_cgm_vec2<24>, dim3((unsigned)L.blocks), dim3(L.threads), 0, ctx->stream, g, s, r, sol, ps, sstride,
-                     (const CgmState*)states, L.s, L.nchunks, ctx->partial);
-  NQ_HIP(hipGetLastError());
-  prof_end(ctx, ev);
-  return launch_cgm_finalize(ctx, states, 1, 2, 1.0);
-}
-
-int launch_cgm_vec3(nq_ctx* ctx, const SpinorView& r, const SpinorView& p, const SpinorView& ps, int64_t sstride,
-                    void* states)
-{
-  const Geo& g = ctx->geo;
-  const Launch L = launch_shape(g, 1);
-  if (r.ncomp != 24) return fail(NQ_EINVAL, "cgm vectors: lx spincolor fields expected");
-  hipEvent_t ev = nullptr;
-  prof_begin(ctx, "cgm_vec3", 0.0, &ev);
-  hipLaunchKernelGGL(k_cgm_vec3<24>, dim3((unsigned)L.blocks), dim3(L.threads), 0, ctx->stream, g, r, p, ps, sstride,
-                     (const CgmState*)states, L.s);
+  // average over the two kinds of iteration
+  prof_begin(ctx, "cgm_vec", 16.0 * (4 + 2 * nshift) * (double)n, &ev);
+  hipLaunchKernelGGL(k_cgm_vec, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, n, (const double2*)r.data,
+                     (double2*)rprev.data, (double2*)p.data, (double2*)sol.data, (double2*)ps.data, sstride,
+                     (const CgmState*)states);
   NQ_HIP(hipGetLastError());
   prof_end(ctx, ev);
   return NQ_OK;

@@ -893,7 +893,7 @@ static bool launch_persistent(nq_ctx* ctx, int op, const SpinorView& out, const 
     const int64_t nblk = (L.nchunks + 3) / 4, slots = (int64_t)ctx->ncu * persist_per_cu<SP, LK, MODE, XP, CLV>();
     if (slots < 1 || nblk < 2 * slots) return false;
     NQ_HOP_LAUNCH((k_tm_hop_lds_p<SP, LK, MODE, XP, CLV>), dim3((unsigned)slots), dim3(256),
-                       ctx->geo, op, out, in, U, anis, anis != 1.0 ? 1 : 0, epi, nblk, L.nchunks, ctx->partial);
+                       ctx->geo, op, out, in, U, anis, anis != 1.0 ? 1 : 0, epi, nblk, L.nchunks, ctx->partial + epi.part0);
     return true;
   } else {
     (void)ctx; (void)op; (void)out; (void)in; (void)U; (void)anis; (void)epi; (void)L;
@@ -909,7 +909,9 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
   const int nr = epi.nrhs;
   if (nr < 1 || nr > 16) return fail(NQ_EINVAL, "tm hop: right-hand sides per launch must be 1..16");
   const Launch L = launch_shape(g, nr);
-  if (L.nchunks * nr > ctx->max_partials) return fail(NQ_EINVAL, "tm hop: reduction scratch too small");
+  if (epi.part0 != 0 && (nr != 1 || epi.batched || epi.fin != FIN_PARTIAL))
+    return fail(NQ_EINVAL, "tm hop: a partial offset needs one right-hand side and FIN_PARTIAL");
+  if (epi.part0 < 0 || epi.part0 + L.nchunks * nr > ctx->max_partials) return fail(NQ_EINVAL, "tm hop: reduction scratch too small");
   if constexpr (MODE != 3 && CLV == 0) {
     if (epi.batched || nr > 1) {
       // register-blocked right-hand sides (always for batched solves, so that a
@@ -945,16 +947,16 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
   if (lds_ok && !fold_here && launch_persistent<SP, LK, MODE, XP, CLV>(ctx, op, out, in, U, anis, epi, L)) {
   } else if (lds_ok && keep) {
     NQ_HOP_LAUNCH((k_tm_hop_lds<SP, LK, MODE, XP, CLV, 0>), grid, blk, g, op, out, in, U, anis, ua, ke, L.s, L.nchunks,
-                  ctx->partial);
+                  ctx->partial + epi.part0);
   } else if (lds_ok) {
     NQ_HOP_LAUNCH((k_tm_hop_lds<SP, LK, MODE, XP, CLV, kNT>), grid, blk, g, op, out, in, U, anis, ua, ke, L.s,
-                  L.nchunks, ctx->partial);
+                  L.nchunks, ctx->partial + epi.part0);
   } else if (keep) {
     NQ_HOP_LAUNCH((k_tm_hop<SP, LK, MODE, XP, CLV, 0>), grid, blk, g, op, out, in, U, anis, ua, ke, L.s, L.nchunks,
-                  ctx->partial);
+                  ctx->partial + epi.part0);
   } else {
     NQ_HOP_LAUNCH((k_tm_hop<SP, LK, MODE, XP, CLV, kNT>), grid, blk, g, op, out, in, U, anis, ua, ke, L.s, L.nchunks,
-                  ctx->partial);
+                  ctx->partial + epi.part0);
   }
   prof_end_ext(ctx);
   NQ_HIP(hipGetLastError());

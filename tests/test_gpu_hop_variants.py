@@ -69,3 +69,23 @@ def test_f16_solves_with_phases(L, theta):
             assert all(r["rc"] == nq.NQ_OK for r in res)
             for i in range(n):
                 assert rel_l2(fx[i].download(), ref[i]) < 1e-10, (prec, i)
+
+
+# every iteration count up to six: the shift vectors are updated in pairs of iterations,
+# and the end comes on a first or a second one
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6])
+def test_q2_multi_mass_iterates(n):
+    L = (6, 4, 2, 4)
+    conf = conf_of(L, 53, [1.0, 0, 0, 0])
+    geo = orc.Geom(L)
+    masses, residues = [0.1, 0.3, 0.9, 3.0], [1e-24, 1e-3, 1e-2, 1e-1]  # some stop on the way
+    src = nq.source_lx(L, 80)
+    ref = geo.tmQ2_cgm(conf, 0.12, masses, n, residues, src)[0]
+    with nq.Ctx(L) as ctx:
+        g = nq.Gauge(ctx, lx=conf)
+        sols = [ctx.field(nq.SPINCOLOR, nq.LX) for _ in masses]
+        st = nq.tmQ2_cgm(ctx, g, 0.12, masses, n, residues, sols, ctx.field(nq.SPINCOLOR, nq.LX, src))
+        assert st["iters"] == n
+        for k in range(4):
+            assert rel_l2(sols[k].download(), ref[k]) < 1e-12, k
+
