@@ -502,6 +502,152 @@ static int persist_per_cu()
   return occ;
 }
 
+// ---------------------------------------------------------------- directions split over wavefronts
+// FP64, one right-hand side: the four wavefronts of a workgroup take the four directions
+// (two slots each) of the same 64 sites, exchange their partial sums through LDS and
+// finish one spin each: wavefront w sums the four directions of spin w in the order
+// t, x, y, z and runs the epilogue on its three components.  A small lattice is bound by
+// the latency of one thread's chain (eight slots of loads and 1320 flops: 10 us on 8^4,
+// of which 3 us are an empty launch's); four times the wavefronts with a quarter of the
+// chain take it to 4.6 us (K K^+ at 12x6x10x14 66 -> 34 us, the FP64 solve at 8^3x16 4.74
+// -> 2.76 ms), and on middle lattices they put more loads in flight (16^3x32 5.4 TB/s of
+// compulsory bytes from the memory-side cache).  130 registers, three workgroups a CU;
+// held to 128 for four it spills and was slower (16^3x32 K K^+ 90 -> 96 us).
+template <int LK, int MU, int CP>
+__device__ __forceinline__ void split_direction(const Geo& g, const Site& s, uint32_t e, const SpinorView& in,
+                                                const void* ub, const double* det, double anis, bool ua,
+                                                double2 (*xch)[3][3][64], int lane, cx<double> own[3])
+{
+  cx<double> o[12];
+#pragma unroll
+  for (int k = 0; k < 12; k++) o[k] = mk(0.0, 0.0);
+  hop_slot<SP_F64, LK, double, MU, true, false, CP>(g, s, e, in, 0, ub, det, 0u, anis, ua, o);
+  hop_slot<SP_F64, LK, double, MU, false, false, CP>(g, s, e, in, 0, ub, det, 0u, anis, ua, o);
+#pragma unroll
+  for (int k = 0; k < 12; k++) {
+    if (k / 3 == MU) own[k % 3] = o[k];
+    else xch[k / 3][MU < k / 3 ? MU : MU - 1][k % 3][lane] = make_double2(o[k].re, o[k].im);
+  }
+}
+
+// three consecutive components of an FP64 field
+template <int CP>
+__device__ __forceinline__ void load3(const SpinorView& v, int64_t stride, uint32_t e, int k0, cx<double> s[3])
+{
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc((const char*)v.data + (int64_t)k0 * stride * 16, 3 * stride * 16);
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    const double2 d = bload_d2<CP>(rs, e * 16u, (uint32_t)(c * stride * 16));
+    s[c] = mk(d.x, d.y);
+  }
+}
+template <int CP>
+__device__ __forceinline__ void store3(const SpinorView& v, int64_t stride, uint32_t e, int k0, const cx<double> s[3])
+{
+#pragma unroll
+  for (int c = 0; c < 3; c++)
+    put<nq_dv2, CP>((nq_dv2*)((char*)v.data + ((int64_t)(k0 + c) * stride + e) * 16), nq_dv2{s[c].re, s[c].im});
+}
+
+template <int LK, int MODE, int CP>
+__global__ void __launch_bounds__(256, 2) k_tm_hop_split(Geo g, int op, SpinorView out, SpinorView in, LinkView U,
+                                                      double anis, int use_anis, HopEpi epi, int64_t nchunks,
+                                                      double* partial)
+{
+  __shared__ double2 xch[4][3][3][64];  // [spin][other direction][colour][site]
+  __shared__ double wsum[4];
+  if constexpr (MODE == 0) {
+    if (fold_finalise(epi, partial, nchunks, (double*)xch)) return;
+  }
+  const CgState* st = epi.st;
+  if (st && rhs_idle(st, epi.pred_reliable)) return;  // uniform: one right-hand side per launch
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t chunk = xcd_block();
+  const bool active = chunk * 64 + lane < g.Vh;
+  // lanes past the end of a partial last chunk compute the last site and drop it
+  const uint32_t e = active ? (uint32_t)(chunk * 64 + lane) : (uint32_t)(g.Vh - 1);
+  const Site s = site_of(g, op, e);
+  const void* ub = U.data[op];
+  const double* det = &U.det[op][0][0];
+  const bool ua = use_anis != 0;
+  cx<double> own[3];
+  if (w == 0) split_direction<LK, 0, CP>(g, s, e, in, ub, det, anis, ua, xch, lane, own);
+  else if (w == 1) split_direction<LK, 1, CP>(g, s, e, in, ub, det, anis, ua, xch, lane, own);
+  else if (w == 2) split_direction<LK, 2, CP>(g, s, e, in, ub, det, anis, ua, xch, lane, own);
+  else split_direction<LK, 3, CP>(g, s, e, in, ub, det, anis, ua, xch, lane, own);
+  // the epilogue's fields of spin w, in flight over the barrier
+  const int k0 = 3 * w, hh = w >> 1;
+  cx<double> a1[3], a2[3], xv[3], pv[3], rv[3];
+  if (epi.aux.data) load3<CP>(epi.aux, g.stride, e, k0, a1);
+  if (epi.aux2.data) load3<CP>(epi.aux2, g.stride, e, k0, a2);
+  if constexpr (MODE == 2) {
+    if (epi.x.data) {
+      load3<CP>(epi.x, g.stride, e, k0, xv);
+      load3<CP>(epi.p, g.stride, e, k0, pv);
+    }
+    load3<CP>(epi.r, g.stride, e, k0, rv);
+  }
+  __syncthreads();
+  cx<double> o[3];
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    // directions in order, this wavefront's own in its place
+    cx<double> t[3];
+#pragma unroll
+    for (int m = 0; m < 3; m++) t[m] = mk(xch[w][m][c][lane].x, xch[w][m][c][lane].y);
+    const cx<double> d0 = w == 0 ? own[c] : t[0], d1 = w == 1 ? own[c] : (w == 0 ? t[0] : t[1]),
+                     d2 = w == 2 ? own[c] : (w < 2 ? t[1] : t[2]), d3 = w == 3 ? own[c] : t[2];
+    o[c] = ((d0 + d1) + d2) + d3;
+  }
+  const cx<double> c1 = mk(epi.c1[hh][0], epi.c1[hh][1]), c2 = mk(epi.c2[hh][0], epi.c2[hh][1]),
+                   c3 = mk(epi.c3[hh][0], epi.c3[hh][1]);
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    o[c] = c1 * o[c];
+    if (epi.aux.data) fma_to(o[c], c2, a1[c]);
+    if (epi.aux2.data) fma_to(o[c], c3, a2[c]);
+  }
+  double nrm = 0;
+  if (active) {
+    if constexpr (MODE == 0) {
+      store3<CP>(out, g.stride, e, k0, o);
+    } else if constexpr (MODE == 1) {
+      if (epi.write) store3<CP>(out, g.stride, e, k0, o);
+#pragma unroll
+      for (int c = 0; c < 3; c++) nrm += o[c].re * o[c].re + o[c].im * o[c].im;
+    } else if constexpr (MODE == 2) {
+      // CG tail: x += alpha p (when x is given) ; r -= alpha s ; |r|^2
+      const double alpha = sload(&st->alpha);
+      if (epi.x.data) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          xv[c].re = fma(alpha, pv[c].re, xv[c].re);
+          xv[c].im = fma(alpha, pv[c].im, xv[c].im);
+        }
+        store3<CP>(epi.x, g.stride, e, k0, xv);
+      }
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        rv[c].re = fma(-alpha, o[c].re, rv[c].re);
+        rv[c].im = fma(-alpha, o[c].im, rv[c].im);
+        nrm += rv[c].re * rv[c].re + rv[c].im * rv[c].im;
+      }
+      store3<CP>(epi.r, g.stride, e, k0, rv);
+    } else {
+      // residual tail: r64 = o ; |o|^2
+      store3<CP>(epi.r, g.stride, e, k0, o);
+#pragma unroll
+      for (int c = 0; c < 3; c++) nrm += o[c].re * o[c].re + o[c].im * o[c].im;
+    }
+  }
+  if constexpr (MODE != 0) {
+    nrm = wave_sum(nrm);
+    if (lane == 0) wsum[w] = nrm;
+    __syncthreads();
+    if (threadIdx.x == 0) partial[chunk] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+  }
+}
+
 // ---------------------------------------------------------------- register-blocked RHS
 // One slot of the hop for RB right-hand sides r0..r0+nrb-1 of the same site: the
 // link is loaded once and applied to each right-hand side's projected neighbour.
@@ -840,6 +986,12 @@ inline bool use_lds(int sp, int lk, const Geo& g, bool keep)
   return lk == LK_F32_12 && g.Vh >= (int64_t(1) << 19);
 }
 
+// FP64 hops of one right-hand side split the directions over the wavefronts below 2^18
+// sites per parity, where the persistent kernel does not fill its slots twice.  Split
+// against one thread per site: 8^4 10.3 / 4.6 us, 12x6x10x14 14.5 / 4.7, 24x12^3 16.6 / 7.4,
+// 16^3x32 20.2 / 18.6, 20^3x40 55.0 / 48.6; above, 24^3x48 98 / 103, 28^3x56 177 / 190.
+inline bool use_split(const Geo& g) { return g.Vh < 1024 * kStageSites; }
+
 // Batched FP16 hops run k_tm_hop_rl, except one or two right-hand sides on a lattice that
 // fills the chip twice over with 256-site blocks: there the links of a site serve too few
 // right-hand sides to pay for k_tm_hop_rl's two wavefronts per SIMD (32^3x64: one 100.5
@@ -944,6 +1096,25 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
   const int ua = anis != 1.0 ? 1 : 0;
   const bool keep = links_stay(g, SP, LK, epi);
   const bool lds_ok = nr == 1 && L.s.W == 4 && !(lenv && lenv[0] == '0') && use_lds(SP, LK, g, keep);
+  if constexpr (SP == SP_F64 && XP == SP_F64 && CLV == 0) {
+    if (nr == 1 && use_split(g) && !epi.coef && !(MODE == 3 && epi.rs.data)) {
+      HopEpi ks = epi;
+      fold_here = MODE == 0 && epi.fold_fin != FIN_NONE && epi.st;
+      if (!fold_here) ks.fold_fin = FIN_NONE;
+      const dim3 sg((unsigned)(L.nchunks + (fold_here ? 1 : 0)));
+      if (keep)
+        NQ_HOP_LAUNCH((k_tm_hop_split<LK, MODE, 0>), sg, dim3(256), g, op, out, in, U, anis, ua, ks, L.nchunks,
+                      ctx->partial + epi.part0);
+      else
+        NQ_HOP_LAUNCH((k_tm_hop_split<LK, MODE, kNT>), sg, dim3(256), g, op, out, in, U, anis, ua, ks, L.nchunks,
+                      ctx->partial + epi.part0);
+      prof_end_ext(ctx);
+      NQ_HIP(hipGetLastError());
+      if (epi.fold_fin != FIN_NONE && !fold_here) NQ_TRY(launch_finalize(ctx, 1, epi.st, epi.fold_fin, epi.fold_pred));
+      if (MODE != 0 && epi.fin != FIN_PARTIAL) NQ_TRY(launch_finalize(ctx, nr, epi.st, epi.fin, epi.pred_reliable));
+      return NQ_OK;
+    }
+  }
   if (lds_ok && !fold_here && launch_persistent<SP, LK, MODE, XP, CLV>(ctx, op, out, in, U, anis, epi, L)) {
   } else if (lds_ok && keep) {
     NQ_HOP_LAUNCH((k_tm_hop_lds<SP, LK, MODE, XP, CLV, 0>), grid, blk, g, op, out, in, U, anis, ua, ke, L.s, L.nchunks,

@@ -89,3 +89,22 @@ def test_q2_multi_mass_iterates(n):
         for k in range(4):
             assert rel_l2(sols[k].download(), ref[k]) < 1e-12, k
 
+
+
+def test_persistent_hop_same_bits_large(monkeypatch):
+    """262144 sites per parity, the smallest lattice of the persistent FP64 hop: the hop
+    and a solve have the bits of the one-shot kernel."""
+    L = (16, 32, 32, 32)
+    conf = conf_of(L, 54, [1.0, 0, 0, 0])
+    with nq.Ctx(L) as ctx:
+        g = nq.Gauge(ctx, lx=conf)
+        fi, fo = ctx.field(nq.SPINCOLOR, nq.ODD, gauss_eo(ctx.Vh, 9)), ctx.field(nq.SPINCOLOR, nq.EVEN)
+        fs, fx = ctx.field(nq.SPINCOLOR, nq.LX, nq.source_lx(L, 11)), ctx.field(nq.SPINCOLOR, nq.LX)
+        out = []
+        for mode in ("1", "0"):
+            monkeypatch.setenv("NQ_PERSIST", mode)
+            nq.tm_hop(ctx, g, fo, fi)
+            st = nq.tm_solve_eoprec(ctx, g, 0.16, 0.05, 1000, 1e-14, fx, fs)
+            assert st["rc"] == nq.NQ_OK
+            out.append((fo.download(), fx.download()))
+        assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
