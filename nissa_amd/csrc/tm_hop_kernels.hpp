@@ -25,7 +25,6 @@
 #include <algorithm>
 #include <cstdlib>
 #include <string>
-
 #include "clover_block.hpp"
 
 namespace nq {
@@ -143,17 +142,20 @@ __device__ __forceinline__ void scatter(cx<R> o[12], const cx<R> g0[3], const cx
 }
 
 // lds: staged records of sites [lds_e0, lds_e0 + kStageSites) of `in`, or null
-template <int SP, int LK, class R, int MU, bool FWD, bool PIN, int CP>
+template <int SP, int LK, class R, int MU, bool FWD, bool PIN, int CP, bool STAGED>
 __device__ __forceinline__ void hop_slot(const Geo& g, const Site& s, uint32_t e, const SpinorView& in, int r,
                                          const void* ub, const double* det, unsigned unit, R anis, bool use_anis,
                                          cx<R> o[12], const char* lds = nullptr, uint32_t lds_e0 = 0)
 {
   const uint32_t n = neigh_eo(g, s, MU, FWD);
-  cx<R> h0[3], h1[3];
-  load_projected<SP, R, MU, FWD>(g, in, r, n, lds, lds_e0, h0, h1);
-  cx<R> u[9];
   constexpr int slot = 2 * MU + (FWD ? 0 : 1);
-  LkAcc<LK, R, CP>::load(ub, g.stride, slot, e, det + 2 * slot, u, lk_eb(LK) < 16 && ((unit >> MU) & 1u));
+  // staged: the link's loads first; with the neighbour in LDS or memory (a branch) in
+  // front of them they would be issued only after its wait
+  cx<R> u[9], h0[3], h1[3];
+  if constexpr (STAGED) LkAcc<LK, R, CP>::load_stored(ub, g.stride, slot, e, u);
+  load_projected<SP, R, MU, FWD>(g, in, r, n, STAGED ? lds : nullptr, lds_e0, h0, h1);
+  if constexpr (!STAGED) LkAcc<LK, R, CP>::load_stored(ub, g.stride, slot, e, u);
+  LkAcc<LK, R, CP>::complete(det + 2 * slot, u, lk_eb(LK) < 16 && ((unit >> MU) & 1u));
   cx<R> g0[3], g1[3];
   mat_vec(u, h0, g0);
   mat_vec(u, h1, g1);
@@ -177,19 +179,19 @@ __device__ __forceinline__ void hop_slot(const Geo& g, const Site& s, uint32_t e
 // (PK = 4: two groups of four slots; the persistent FP64 kernel takes PK = 2).  The
 // pins order the schedule only; the arithmetic, and so every bit of the result, is
 // the same for every PK.
-template <int SP, int LK, class R, int PK, int CP>
+template <int SP, int LK, class R, int PK, int CP, bool STAGED>
 __device__ __forceinline__ void hop_site(const Geo& g, const Site& s, uint32_t e, const SpinorView& in, int r,
                                          const void* ub, const double* det, unsigned unit, R anis, bool ua, cx<R> o[12],
                                          const char* lds = nullptr, uint32_t e0 = 0)
 {
-  hop_slot<SP, LK, R, 0, true, (1 % PK) == 0, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
-  hop_slot<SP, LK, R, 0, false, (2 % PK) == 0, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
-  hop_slot<SP, LK, R, 1, true, (3 % PK) == 0, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
-  hop_slot<SP, LK, R, 1, false, (4 % PK) == 0, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
-  hop_slot<SP, LK, R, 2, true, (5 % PK) == 0, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
-  hop_slot<SP, LK, R, 2, false, (6 % PK) == 0, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
-  hop_slot<SP, LK, R, 3, true, (7 % PK) == 0, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
-  hop_slot<SP, LK, R, 3, false, true, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+  hop_slot<SP, LK, R, 0, true, (1 % PK) == 0, CP, STAGED>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+  hop_slot<SP, LK, R, 0, false, (2 % PK) == 0, CP, STAGED>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+  hop_slot<SP, LK, R, 1, true, (3 % PK) == 0, CP, STAGED>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+  hop_slot<SP, LK, R, 1, false, (4 % PK) == 0, CP, STAGED>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+  hop_slot<SP, LK, R, 2, true, (5 % PK) == 0, CP, STAGED>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+  hop_slot<SP, LK, R, 2, false, (6 % PK) == 0, CP, STAGED>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+  hop_slot<SP, LK, R, 3, true, (7 % PK) == 0, CP, STAGED>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+  hop_slot<SP, LK, R, 3, false, true, CP, STAGED>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
 }
 
 template <int SP>
@@ -350,12 +352,15 @@ __global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop(Geo g, i
     cx<R> o[12];
 #pragma unroll
     for (int k = 0; k < 12; k++) o[k] = mk<R>(0, 0);
-    hop_site<SP, LK, R, 4, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o);
+    hop_site<SP, LK, R, 4, CP, false>(g, s, e, in, r, ub, det, unit, anis, ua, o);
     nrm = hop_epilogue<SP, MODE, XP, R, CLV, CP>(g, epi, out, e, r, st, o);
   }
   if constexpr (MODE != 0) store_partial(nrm, partial, nchunks, m.r, m.chunk);
 }
 
+// The accumulators are pinned after every slot for FP16 (76-87 registers instead of 128,
+// five or six wavefronts per SIMD beside the 13 KB of LDS: 32^3x64 hop 88 -> 85 us, FP16
+// links 74 -> 61), after every four slots otherwise (FP32 139 -> 132 us).
 // One right-hand side, neighbours staged in LDS (Stage): the workgroup's four
 // wavefronts cover 256 consecutive output sites (Shape W = 4, NRB = 1).
 template <int SP, int LK, int MODE, int XP, int CLV = 0, int CP = kNT>
@@ -391,7 +396,7 @@ __global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop_lds(Geo 
     cx<R> o[12];
 #pragma unroll
     for (int k = 0; k < 12; k++) o[k] = mk<R>(0, 0);
-    hop_site<SP, LK, R, 4, CP>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+    hop_site<SP, LK, R, SP == SP_F16 ? 1 : 4, CP, true>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
     nrm = hop_epilogue<SP, MODE, XP, R, CLV, CP>(g, epi, out, e, r, st, o);
   }
   if constexpr (MODE != 0) store_partial(nrm, partial, nchunks, m.r, m.chunk);
@@ -463,7 +468,7 @@ __global__ void __launch_bounds__(256, 1) k_tm_hop_lds_p(Geo g, int op, SpinorVi
         cx<R> o[12];
 #pragma unroll
         for (int k2 = 0; k2 < 12; k2++) o[k2] = mk<R>(0, 0);
-        hop_site<SP, LK, R, 2, kNT>(g, s, e, in, 0, ub, det, unit, anis, ua, o, lds, (uint32_t)e0);
+        hop_site<SP, LK, R, 2, kNT, true>(g, s, e, in, 0, ub, det, unit, anis, ua, o, lds, (uint32_t)e0);
         hop_epilogue<SP, MODE, XP, R, CLV>(g, epi, out, e, 0, st, o);
       }
     }
@@ -481,7 +486,7 @@ __global__ void __launch_bounds__(256, 1) k_tm_hop_lds_p(Geo g, int op, SpinorVi
       cx<R> o[12];
 #pragma unroll
       for (int k = 0; k < 12; k++) o[k] = mk<R>(0, 0);
-      hop_site<SP, LK, R, 2, kNT>(g, s, e, in, 0, ub, det, unit, anis, ua, o, lds, e0);
+      hop_site<SP, LK, R, 2, kNT, true>(g, s, e, in, 0, ub, det, unit, anis, ua, o, lds, e0);
       nrm = hop_epilogue<SP, MODE, XP, R, CLV>(g, epi, out, e, 0, st, o);
     }
     if constexpr (MODE != 0) store_partial(nrm, partial, nchunks, 0, cb * 4 + wave);
@@ -521,8 +526,8 @@ __device__ __forceinline__ void split_direction(const Geo& g, const Site& s, uin
   cx<double> o[12];
 #pragma unroll
   for (int k = 0; k < 12; k++) o[k] = mk(0.0, 0.0);
-  hop_slot<SP_F64, LK, double, MU, true, false, CP>(g, s, e, in, 0, ub, det, 0u, anis, ua, o);
-  hop_slot<SP_F64, LK, double, MU, false, false, CP>(g, s, e, in, 0, ub, det, 0u, anis, ua, o);
+  hop_slot<SP_F64, LK, double, MU, true, false, CP, false>(g, s, e, in, 0, ub, det, 0u, anis, ua, o);
+  hop_slot<SP_F64, LK, double, MU, false, false, CP, false>(g, s, e, in, 0, ub, det, 0u, anis, ua, o);
 #pragma unroll
   for (int k = 0; k < 12; k++) {
     if (k / 3 == MU) own[k % 3] = o[k];
@@ -974,17 +979,12 @@ inline bool links_stay(const Geo& g, int sp, int lk, const HopEpi& epi)
 }
 
 // Neighbours staged in LDS (k_tm_hop_lds) for one right-hand side: FP64 always (4 % at
-// 32^3x64); FP32 when its links are streamed (solve at 24^3x48 19.1 -> 17.6 ms, 32^3x64
-// 51.2 -> 49.9; 16^3x32, links kept: hop 10.6 -> 12.9 us); FP16 with FP32 links from 2^19
-// sites per parity up (28^3x56 23.8 -> 23.3 ms, 32^3x64 37.3 -> 35.9; 24^3x48 14.1 ->
-// 14.4); never with FP16 links (24^3x48 hop 28 -> 38 us: its 128 registers and the
-// staging leave too few wavefronts).
-inline bool use_lds(int sp, int lk, const Geo& g, bool keep)
-{
-  if (sp == SP_F64) return true;
-  if (sp == SP_F32) return !keep;
-  return lk == LK_F32_12 && g.Vh >= (int64_t(1) << 19);
-}
+// 32^3x64), the sloppy precisions when the links are streamed: unstaged against staged,
+// FP32 54.4 / 49.8 us at 24^3x48 and 139 / 132 at 32^3x64; FP16 34.6 / 33.4 and 91 / 85;
+// FP16 links at 32^3x64 74.8 / 61.3.  With the links in the memory-side cache the staging
+// round trip is not paid back: 16^3x32 FP32 10.7 / 12.0 us, FP16 9.4 / 10.1, FP16 links
+// 9.1 / 9.7; 24^3x48, FP16 links 25.5 / 25.6.
+inline bool use_lds(int sp, bool keep) { return sp == SP_F64 || !keep; }
 
 // FP64 hops of one right-hand side split the directions over the wavefronts below 2^18
 // sites per parity, where the persistent kernel does not fill its slots twice.  Split
@@ -1095,7 +1095,7 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
   const dim3 grid((unsigned)(L.blocks + (fold_here ? 1 : 0))), blk(L.threads);
   const int ua = anis != 1.0 ? 1 : 0;
   const bool keep = links_stay(g, SP, LK, epi);
-  const bool lds_ok = nr == 1 && L.s.W == 4 && !(lenv && lenv[0] == '0') && use_lds(SP, LK, g, keep);
+  const bool lds_ok = nr == 1 && L.s.W == 4 && !(lenv && lenv[0] == '0') && use_lds(SP, keep);
   if constexpr (SP == SP_F64 && XP == SP_F64 && CLV == 0) {
     if (nr == 1 && use_split(g) && !epi.coef && !(MODE == 3 && epi.rs.data)) {
       HopEpi ks = epi;
