@@ -123,6 +123,29 @@ __global__ void __launch_bounds__(256) k_dot(BlasArgs A, SpinorView a, SpinorVie
   store_partial(acc, A.partial, A.nchunks, m.r, m.chunk);
 }
 
+// The finalisation of |r|^2 (A.fin: FIN_RR or FIN_RR_SLOPPY) carried out by every workgroup
+// of a one-source p update for itself: the sum of the chunk partials (same bits as
+// k_finalize's), beta, and whether the source stops or waits for a reliable update, from
+// a state that nobody writes in this launch except rr_new and `pending`, which nobody
+// reads; FIN_PAP (or k_cg_commit) records it.  Returns false when p stays as it is.
+__device__ __forceinline__ bool rr_inline(const BlasArgs& A, double* vl, double* beta)
+{
+  CgState* s = A.st;
+  double tot = block_sum_partials_256(A.partial, A.nchunks, vl);
+  __syncthreads();
+  if (threadIdx.x == 0) vl[0] = tot;
+  __syncthreads();
+  tot = vl[0];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    s->rr_new = tot;
+    s->pending = A.fin;
+  }
+  *beta = tot / s->rr;
+  const bool last = s->iter + 1 >= s->niter;
+  if (A.fin == FIN_RR) return !(isnan(*beta) || !(tot >= s->target) || last);
+  return !(isnan(tot) || sqrt(tot) < s->delta * s->r0 || tot < s->target || last);
+}
+
 // p = r + beta p, beta from state[r]; skipped once that right-hand side is done or
 // while it waits for a reliable update.  With x given, first x += alpha p (the CG
 // solution update moved out of the matvec tail, so that p is read once per
@@ -132,8 +155,15 @@ __global__ void __launch_bounds__(256) k_pupdate(BlasArgs A, SpinorView p, Spino
 {
   const Map m = map_thread(A.s, A.g.Vh);
   const CgState* s = A.st + m.r;
-  if (s->done || !m.active || (A.pred == 2 ? !s->reliable : s->reliable)) return;
-  const double beta = s->beta;
+  if (s->done || (A.pred == 2 ? !s->reliable : s->reliable)) return;  // uniform per right-hand side
+  double beta;
+  if (A.fin != FIN_NONE) {
+    __shared__ double vl[1024];
+    if (!rr_inline(A, vl, &beta)) return;  // one right-hand side: uniform over the workgroup
+  } else {
+    beta = s->beta;
+  }
+  if (!m.active) return;
   cx<double> pv[NC], rv[NC];
   load_any<NC>(p, A.g.stride, m.e, pv, m.r);
   load_any<NC>(r, A.g.stride, m.e, rv, m.r);
@@ -167,12 +197,22 @@ __global__ void __launch_bounds__(256) k_pupdate_pair(BlasArgs A, SpinorView pin
 {
   const Map m = map_thread(A.s, A.g.Vh);
   const CgState* s = A.st + m.r;
-  if (s->done || !m.active || s->reliable) return;
-  const double beta = s->beta;
+  if (s->done || s->reliable) return;
+  double beta;
+  bool xstep;
+  if (A.fin != FIN_NONE) {
+    __shared__ double vl[1024];
+    if (!rr_inline(A, vl, &beta)) return;  // uniform over the workgroup
+    xstep = s->xlag != 0;  // the xstep that recording this finalisation will set
+  } else {
+    beta = s->beta;
+    xstep = s->xstep != 0;
+  }
+  if (!m.active) return;
   cx<double> pv[NC], rv[NC];
   load_any<NC>(pin, A.g.stride, m.e, pv, m.r);
   load_any<NC>(r, A.g.stride, m.e, rv, m.r);
-  if (x.data && s->xstep) {
+  if (x.data && xstep) {
     const double a0 = s->alpha_prev, a1 = s->alpha;
     cx<double> xv[NC], qv[NC];
     load_any<NC>(x, A.g.stride, m.e, xv, m.r);
@@ -403,11 +443,13 @@ int launch_dot(nq_ctx* ctx, const SpinorView& a, const SpinorView& b, int fin, C
 }
 
 int launch_cg_pupdate(nq_ctx* ctx, const SpinorView& p, const SpinorView& r, CgState* st, int nr, int pred,
-                      const SpinorView& x)
+                      const SpinorView& x, int fin)
 {
   BlasArgs A;
   Launch L;
-  NQ_TRY(make_args(ctx, nr, st, FIN_NONE, pred == 2 ? 2 : 1, &A, &L));
+  NQ_TRY(make_args(ctx, nr, st, fin, pred == 2 ? 2 : 1, &A, &L));
+  if (fin != FIN_NONE && (nr != 1 || L.threads != 256 || pred != 1 || (fin != FIN_RR && fin != FIN_RR_SLOPPY)))
+    return fail(NQ_EINVAL, "pupdate: finalisation %d needs one right-hand side", fin);
   if (x.data && x.ncomp != p.ncomp) return fail(NQ_EINVAL, "pupdate: component mismatch");
   hipEvent_t ev = nullptr;
   const double xb = x.data ? 2.0 * site_bytes(x) : 0.0;
@@ -419,6 +461,21 @@ int launch_cg_pupdate(nq_ctx* ctx, const SpinorView& p, const SpinorView& r, CgS
   else hipLaunchKernelGGL(k_pupdate<3>, grid, blk, 0, ctx->stream, A, p, r, x);
   NQ_HIP(hipGetLastError());
   prof_end(ctx, ev);
+  return NQ_OK;
+}
+
+__global__ void k_cg_commit(CgState* st)
+{
+  if (!st->pending) return;
+  const int f = st->pending;
+  st->pending = FIN_NONE;
+  finalize(st, f, st->rr_new);
+}
+
+int launch_cg_commit(nq_ctx* ctx, CgState* st)
+{
+  hipLaunchKernelGGL(k_cg_commit, dim3(1), dim3(1), 0, ctx->stream, st);
+  NQ_HIP(hipGetLastError());
   return NQ_OK;
 }
 
@@ -436,11 +493,13 @@ int launch_clear_reliable(nq_ctx* ctx, CgState* st, int nr)
 }
 
 int launch_cg_pupdate_pair(nq_ctx* ctx, const SpinorView& p_in, const SpinorView& p_out, const SpinorView& r,
-                           CgState* st, const SpinorView& x)
+                           CgState* st, const SpinorView& x, int fin)
 {
   BlasArgs A;
   Launch L;
-  NQ_TRY(make_args(ctx, 1, st, FIN_NONE, 1, &A, &L));
+  NQ_TRY(make_args(ctx, 1, st, fin, 1, &A, &L));
+  if (fin != FIN_NONE && (L.threads != 256 || (fin != FIN_RR && fin != FIN_RR_SLOPPY)))
+    return fail(NQ_EINVAL, "pupdate pair: bad finalisation %d", fin);
   if (p_in.data == p_out.data) return fail(NQ_EINVAL, "pupdate pair: p_in and p_out must differ");
   if (p_in.ncomp != p_out.ncomp || (x.data && x.ncomp != p_in.ncomp)) return fail(NQ_EINVAL, "pupdate pair: component mismatch");
   hipEvent_t ev = nullptr;

@@ -486,8 +486,16 @@ __device__ __forceinline__ double wave_sum(double v)
   return v;
 }
 
+// One recurrence of the CG / mixed CG.  FIN_PAP first records a finalisation that the p
+// update left pending; when that one stops the source or raises `reliable`, alpha stays.
 __device__ inline void finalize(CgState* st, int fin, double total)
 {
+  if (fin == FIN_PAP && st->pending) {
+    const int f = st->pending;
+    st->pending = FIN_NONE;
+    finalize(st, f, st->rr_new);
+    if (st->done || st->reliable) return;
+  }
   switch (fin) {
   case FIN_STORE0: st->extra[0] = total; break;
   case FIN_STORE1: st->extra[1] = total; break;

@@ -99,7 +99,9 @@ struct CgState {
   double true_rr;       // last FP64 residual
   double extra[6];
   double alpha_prev;    // alpha of the previous iteration (paired x updates)
-  int iter, niter, done, reliable, nreliable, nan, mixed, flags;
+  // pending: a finalisation (Fin) of rr_new that the p update has acted on (launch_cg_pupdate
+  // with fin) and that the next FIN_PAP finalisation or launch_cg_commit records
+  int iter, niter, done, reliable, nreliable, nan, mixed, pending;
   // paired x updates of the one-source mixed CG: xlag = the last p update left its
   // alpha p term to the next one; xstep = the coming p update applies both terms
   int xlag, xstep;
@@ -422,7 +424,14 @@ int launch_dot(nq_ctx* ctx, const SpinorView& a, const SpinorView& b, int fin, C
 // p = r + beta p; pred 1: skip done or reliable-pending right-hand sides; 2: only the
 // reliable-pending ones (after FIN_RR_TRUE_HOLD)
 int launch_cg_pupdate(nq_ctx* ctx, const SpinorView& p, const SpinorView& r, CgState* st, int nr = 1, int pred = 1,
-                      const SpinorView& x = SpinorView());
+                      const SpinorView& x = SpinorView(), int fin = FIN_NONE);
+// record a finalisation left pending by a p update
+int launch_cg_commit(nq_ctx* ctx, CgState* st);
+// whether every workgroup of the one-source p update sums the chunk partials of |r|^2
+// itself (fin of launch_cg_pupdate and launch_cg_pupdate_pair: FIN_RR or FIN_RR_SLOPPY)
+// instead of a finalisation launched before it: the sum of up to 1024 partials is four
+// loads a thread, a launch and its gap 6-8 us
+inline bool fold_rr(const Geo& g) { return g.Vh <= 1024 * 64; }
 // state[i].reliable = 0 for i < nr
 int launch_clear_reliable(nq_ctx* ctx, CgState* st, int nr);
 int launch_reliable_accum(nq_ctx* ctx, const SpinorView& x64, const SpinorView& xs, CgState* st, int nr = 1,
@@ -431,7 +440,7 @@ int launch_reliable_accum(nq_ctx* ctx, const SpinorView& x64, const SpinorView& 
 // reliable-pending); with x, when the state's xstep is set, first
 // x += alpha_prev p_prev + alpha p_in, p_prev being p_out's old content
 int launch_cg_pupdate_pair(nq_ctx* ctx, const SpinorView& p_in, const SpinorView& p_out, const SpinorView& r,
-                           CgState* st, const SpinorView& x = SpinorView());
+                           CgState* st, const SpinorView& x = SpinorView(), int fin = FIN_NONE);
 int launch_convert(nq_ctx* ctx, const SpinorView& out, const SpinorView& in, int nr = 1,
                    CgState* st = nullptr, int pred = 0);
 int launch_zero(nq_ctx* ctx, const SpinorView& v, int nr = 1);

@@ -243,6 +243,7 @@ static int cg_kernsq_f64(const TmSetup& S, double mu, int niter, double residue,
   NQ_TRY(launch_convert(ctx, p, r));
   NQ_TRY(get_states(ctx, 0, 1));
   const double rr0 = ctx->state_host[0].rr;
+  const bool fold = fold_rr(ctx->geo);
   int chunk = 8, launched = 0;
   while (!ctx->state_host[0].done) {
     for (int i = 0; i < chunk; i++) {
@@ -252,21 +253,25 @@ static int cg_kernsq_f64(const TmSetup& S, double mu, int niter, double residue,
       HopEpi b1 = epi_kout(S.kappa, -mu, p);
       b1.mode = 1;
       b1.st = st;
-      b1.fin = FIN_PAP;
+      b1.fin = FIN_PARTIAL;
       NQ_TRY(launch_tm_hop(ctx, NQ_ODD, t1, tmp, S.U, S.anis, b1));
+      // alpha from the partials of <p, K K^+ p>, where the kernel takes it along in an
+      // extra workgroup of this hop
       HopEpi a2 = epi_inv_dee(S.kappa, mu);
       a2.st = st;
+      a2.fold_fin = FIN_PAP;
       NQ_TRY(launch_tm_hop(ctx, NQ_EVEN, tmp, t1, S.U, S.anis, a2));
       HopEpi b2 = epi_kout(S.kappa, mu, t1);
       b2.mode = 2;
       b2.st = st;
-      b2.fin = FIN_RR;
+      b2.fin = fold ? FIN_PARTIAL : FIN_RR;
       b2.x = x;
       b2.p = p;
       b2.r = r;
       NQ_TRY(launch_tm_hop(ctx, NQ_ODD, none, tmp, S.U, S.anis, b2));
-      NQ_TRY(launch_cg_pupdate(ctx, p, r, st));
+      NQ_TRY(launch_cg_pupdate(ctx, p, r, st, 1, 1, SpinorView(), fold ? FIN_RR : FIN_NONE));
     }
+    if (fold) NQ_TRY(launch_cg_commit(ctx, st));
     launched += chunk;
     NQ_TRY(get_states(ctx, 0, 1));
     const CgState& h = ctx->state_host[0];
@@ -346,6 +351,7 @@ static int cg_kernsq_mixed(const TmSetup& S64, const TmSetup& Ss, int sp, double
   // The sloppy iterations idle (device flag) once a reliable update is due; the host
   // polls after chunks sized from the observed convergence rate to end where the
   // next update is expected, and then runs the FP64 update unconditionally.
+  const bool fold = fold_rr(ctx->geo);
   int chunk = 8, launched = 0;
   while (!ctx->state_host[0].done) {
     // iteration j of the solve uses p[j % 2]; the chunk starts at the device's count
@@ -374,15 +380,16 @@ static int cg_kernsq_mixed(const TmSetup& S64, const TmSetup& Ss, int sp, double
       HopEpi b2 = epi_kout(Ss.kappa, mu, t1s);
       b2.mode = 2;
       b2.st = st;
-      b2.fin = FIN_RR_SLOPPY;
+      b2.fin = fold ? FIN_PARTIAL : FIN_RR_SLOPPY;
       b2.pred_reliable = 2;
       b2.p = p;
       b2.r = rs;
       NQ_TRY(launch_tm_hop(ctx, NQ_ODD, none, tmps, Ss.U, Ss.anis, b2));
       // p_next = rs + beta p and, every other iteration, xs += the two iterations'
       // alpha p terms
-      NQ_TRY(launch_cg_pupdate_pair(ctx, p, pn, rs, st, xs));
+      NQ_TRY(launch_cg_pupdate_pair(ctx, p, pn, rs, st, xs, fold ? FIN_RR_SLOPPY : FIN_NONE));
     }
+    if (fold) NQ_TRY(launch_cg_commit(ctx, st));
     launched += chunk;
     NQ_TRY(get_states(ctx, 0, 1));
     if (ctx->state_host[0].reliable && !ctx->state_host[0].done) {

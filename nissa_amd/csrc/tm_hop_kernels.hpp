@@ -1115,7 +1115,8 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
       return NQ_OK;
     }
   }
-  if (lds_ok && !fold_here && launch_persistent<SP, LK, MODE, XP, CLV>(ctx, op, out, in, U, anis, epi, L)) {
+  if (lds_ok && launch_persistent<SP, LK, MODE, XP, CLV>(ctx, op, out, in, U, anis, epi, L)) {
+    fold_here = false;
   } else if (lds_ok && keep) {
     NQ_HOP_LAUNCH((k_tm_hop_lds<SP, LK, MODE, XP, CLV, 0>), grid, blk, g, op, out, in, U, anis, ua, ke, L.s, L.nchunks,
                   ctx->partial + epi.part0);
