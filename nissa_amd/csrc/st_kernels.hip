@@ -505,84 +505,109 @@ __global__ void __launch_bounds__(256) k_cgm_update(Geo g, SpinorView rv, Spinor
 
 enum { FIN_CGM_PAP = 1, FIN_CGM_RFRF = 2 };
 
-// recurrences of cgm_invert_template_threaded.hpp:118-141 (pap) and :183-252 (rfrf)
+// recurrences of cgm_invert_template_threaded.hpp:118-141 (pap) and :183-252 (rfrf),
+// one shift per lane of a wavefront (all lanes call it with the same total): the shifts
+// of a serial loop cost a chain of memory round trips and FP64 divisions each, 7.7 us a
+// finalisation with 12 shifts, 7 % of a multi-shift iteration at 24^3x48
 __device__ inline void cgm_finalize(CgmState* s, int fin, double total, double pap_scale)
 {
+  const int k = threadIdx.x & 63;
+  const bool mine = k < s->nshift;
+  const bool ran = mine && s->run[k];
   if (fin == FIN_CGM_PAP) {
-    const double pap = pap_scale * total;
-    s->pap = pap;
-    s->betap = s->betaa;
-    s->betaa = -s->rr / pap;
-    for (int k = 0; k < s->nshift; k++) {
-      if (!s->run[k]) continue;
-      const double ratio = s->betap / (s->betaa * s->alpha * (1 - s->zas[k] / s->zps[k]) +
-                                       s->betap * (1 - s->shift[k] * s->betaa));
-      if (isnan(ratio)) { s->nan = 1; s->done = 1; }
+    const double pap = pap_scale * total, betap = s->betaa, betaa = -s->rr / pap;
+    bool bad = false;
+    if (ran) {
+      const double ratio =
+          betap / (betaa * s->alpha * (1 - s->zas[k] / s->zps[k]) + betap * (1 - s->shift[k] * betaa));
+      bad = isnan(ratio);
       s->zfs[k] = s->zas[k] * ratio;
       s->betas_prev[k] = s->betas[k];
-      s->betas[k] = s->betaa * ratio;
+      s->betas[k] = betaa * ratio;
     }
-  } else {
-    const double rfrf = total;
-    s->rfrf = rfrf;
-    s->alpha = rfrf / s->rr;
-    for (int k = 0; k < s->nshift; k++) {
-      if (!s->run[k]) continue;
-      s->alphas[k] = s->alpha * s->zfs[k] * s->betas[k] / (s->zas[k] * s->betaa);
-      s->zps[k] = s->zas[k];
-      s->zas[k] = s->zfs[k];
+    const bool nan = __ballot(bad) != 0;
+    if (k == 0) {
+      s->pap = pap;
+      s->betap = betap;
+      s->betaa = betaa;
+      if (nan) { s->nan = 1; s->done = 1; }
     }
-    if (s->lx)
-      for (int k = 0; k < s->nshift; k++) {
-        if (!s->vlag) {  // this iteration may stay pending
-          s->b1[k] = s->betas[k];
-          s->z1[k] = s->zfs[k];
-          s->a1[k] = s->alphas[k];
-          s->ran1[k] = s->run[k];
-        }
-        s->ran2[k] = s->run[k];
-      }
-    s->rr = rfrf;
-    s->iter += 1;
-    // the C2 just run left its sol_k terms when lag was clear (the next C2 applies
-    // them); a shift that stops, or a source that ends, owes them to the settle kernel
-    const bool owed = s->lag == 0;
-    for (int k = 0; k < s->nshift; k++) {
-      if (!s->run[k]) continue;
-      s->owe[k] = 0;
-      s->res[k] = s->rr * s->zfs[k] * s->zfs[k] / s->b2;
-      if (s->res[k] < s->target[k]) {
-        s->run[k] = 0;
-        s->nrun -= 1;
-        if (owed) s->owe[k] = 1;
-      }
+    return;
+  }
+  const double rfrf = total, alpha = rfrf / s->rr, betaa = s->betaa;
+  const int iter = s->iter + 1, vlag = s->vlag, nrun0 = s->nrun;
+  // the C2 just run left its sol_k terms when lag was clear (the next C2 applies
+  // them); a shift that stops, or a source that ends, owes them to the settle kernel
+  const bool owed = s->lag == 0, mixed = s->mixed != 0, lx = s->lx != 0;
+  bool stop = false;
+  int owe = 0;
+  double res = 0, zfs = 0, shift = 0;
+  if (ran) {
+    zfs = s->zfs[k];
+    shift = s->shift[k];
+    s->alphas[k] = alpha * zfs * s->betas[k] / (s->zas[k] * betaa);
+    s->zps[k] = s->zas[k];
+    s->zas[k] = zfs;
+    res = rfrf * zfs * zfs / s->b2;
+    s->res[k] = res;
+    stop = res < s->target[k];
+    if (stop && owed) owe = 1;
+  }
+  if (lx && mine) {
+    if (!vlag) {  // this iteration may stay pending
+      s->b1[k] = s->betas[k];
+      s->z1[k] = s->zfs[k];
+      s->a1[k] = s->alphas[k];
+      s->ran1[k] = ran;
     }
-    if (isnan(rfrf)) { s->nan = 1; s->done = 1; }
-    if (s->nrun <= 0 || s->iter >= s->niter) s->done = 1;
-    if (s->done && owed)
-      for (int k = 0; k < s->nshift; k++)
-        if (s->run[k]) s->owe[k] = 1;
-    if (s->mixed && !s->done) {
-      int kr = -1;
-      for (int k = 0; k < s->nshift; k++)
-        if (s->run[k] && (kr < 0 || s->shift[k] < s->shift[kr])) kr = k;
-      s->kref = kr;
-      if (kr >= 0 && s->res[kr] < s->delta2 * s->rel_ref) s->reliable = 1;
+    s->ran2[k] = ran;
+  }
+  const bool runs = ran && !stop;
+  const int nrun = nrun0 - __popcll(__ballot(stop));
+  const bool nan = isnan(rfrf);
+  const bool done = nan || nrun <= 0 || iter >= s->niter;
+  if (done && owed && runs) owe = 1;
+  bool reliable = false;
+  int kref = s->kref;
+  if (mixed && !done) {
+    // the running shift with the smallest shift (the first of equal ones)
+    double v = runs ? shift : INFINITY, rv = res;
+    int kr = runs ? k : 64;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const double v2 = __shfl_xor(v, off, 64), rv2 = __shfl_xor(rv, off, 64);
+      const int k2 = __shfl_xor(kr, off, 64);
+      if (k2 < 64 && (kr == 64 || v2 < v || (v2 == v && k2 < kr))) { v = v2; rv = rv2; kr = k2; }
     }
-    // before a reliable update C3 applies the running shifts' owed terms
-    if (s->reliable && owed)
-      for (int k = 0; k < s->nshift; k++)
-        if (s->run[k]) s->owe[k] = 2;
-    // C3 leaves the ps_k update to the next C2 unless the source stops here or a
-    // reliable update (which replaces r) comes first
-    s->pend = !s->done && !s->reliable;
-    s->lag = owed && s->pend;
-    if (s->lx) {
-      // the vector update of this iteration (CgmState::vmode)
-      if (s->vlag) s->vmode = 2;
-      else s->vmode = s->done ? 3 : 1;
-      s->vlag = s->vmode == 1;
-    }
+    kref = kr < 64 ? kr : -1;
+    reliable = kr < 64 && rv < s->delta2 * s->rel_ref;
+  }
+  // before a reliable update C3 applies the running shifts' owed terms
+  if (reliable && owed && runs) owe = 2;
+  if (ran) {
+    s->owe[k] = owe;
+    if (stop) s->run[k] = 0;
+  }
+  if (k != 0) return;
+  s->rfrf = rfrf;
+  s->alpha = alpha;
+  s->rr = rfrf;
+  s->iter = iter;
+  s->nrun = nrun;
+  s->kref = kref;
+  if (nan) s->nan = 1;
+  if (done) s->done = 1;
+  if (reliable) s->reliable = 1;
+  // C3 leaves the ps_k update to the next C2 unless the source stops here or a
+  // reliable update (which replaces r) comes first
+  const int pend = !done && !reliable;
+  s->pend = pend;
+  s->lag = owed && pend;
+  if (lx) {
+    // the vector update of this iteration (CgmState::vmode)
+    const int vmode = vlag ? 2 : (done ? 3 : 1);
+    s->vmode = vmode;
+    s->vlag = vmode == 1;
   }
 }
 
@@ -599,7 +624,7 @@ __global__ void __launch_bounds__(1024) k_cgm_finalize(const double* partial, in
     return;
   }
   const double tot = block_sum_partials(partial + (int64_t)blockIdx.x * nchunks, nchunks, vl);
-  if (threadIdx.x == 0) cgm_finalize(s, fin, tot, pap_scale);
+  if (threadIdx.x < 64) cgm_finalize(s, fin, tot, pap_scale);
 }
 
 // ------------------------------------------------------------------ persistent CGM
@@ -686,7 +711,7 @@ __device__ __forceinline__ void cgm_finalize_block(CgmState* s, const double* pr
     return;
   }
   const double tot = block_sum_partials_256(pr, nchunks, vl);
-  if (threadIdx.x == 0) cgm_finalize(s, fin, tot, pap_scale);
+  if (threadIdx.x < 64) cgm_finalize(s, fin, tot, pap_scale);
 }
 
 template <int SP, int LK, int RB>
@@ -1010,8 +1035,8 @@ __global__ void __launch_bounds__(1024) k_cgm_finalize_lx(const double* partial,
     return;
   }
   const double tot = block_sum_partials(partial, nparts, vl);
+  if (threadIdx.x < 64) cgm_finalize(s, fin, tot, 1.0);
   if (threadIdx.x == 0) {
-    cgm_finalize(s, fin, tot, 1.0);
     mirror->alpha = -s->betaa;
     mirror->done = s->done;
   }
