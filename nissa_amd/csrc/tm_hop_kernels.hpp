@@ -653,6 +653,62 @@ __global__ void __launch_bounds__(256, 2) k_tm_hop_split(Geo g, int op, SpinorVi
   }
 }
 
+// The same split for the sloppy precisions and for the clover epilogues, whose FP16 norms
+// and 6x6 blocks need all components of a site in one thread: the first wavefront sums the
+// four directions and runs the common epilogue.
+template <int SP, int LK, class R, int MU, int CP>
+__device__ __forceinline__ void split_direction_to(const Geo& g, const Site& s, uint32_t e, const SpinorView& in,
+                                                   const void* ub, const double* det, unsigned unit, R anis, bool ua,
+                                                   cx<R> (*xch)[12][64], int lane)
+{
+  cx<R> o[12];
+#pragma unroll
+  for (int k = 0; k < 12; k++) o[k] = mk<R>(0, 0);
+  hop_slot<SP, LK, R, MU, true, false, CP, false>(g, s, e, in, 0, ub, det, unit, anis, ua, o);
+  hop_slot<SP, LK, R, MU, false, false, CP, false>(g, s, e, in, 0, ub, det, unit, anis, ua, o);
+#pragma unroll
+  for (int k = 0; k < 12; k++) xch[MU][k][lane] = o[k];
+}
+
+template <int SP, int LK, int MODE, int XP, int CLV, int CP>
+__global__ void __launch_bounds__(256, 2) k_tm_hop_split_any(Geo g, int op, SpinorView out, SpinorView in, LinkView U,
+                                                             double anis_d, int use_anis, HopEpi epi, int64_t nchunks,
+                                                             double* partial)
+{
+  using R = RealOf<SP>;
+  __shared__ cx<R> xch[4][12][64];  // [direction][component][site]
+  static_assert(sizeof xch >= 8192, "the finalisation needs 1024 doubles");
+  if constexpr (MODE == 0) {
+    if (fold_finalise(epi, partial, nchunks, (double*)xch)) return;
+  }
+  CgState* st = epi.st;
+  if (st && rhs_idle(st, epi.pred_reliable)) return;  // uniform: one right-hand side per launch
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t chunk = xcd_block();
+  const bool active = chunk * 64 + lane < g.Vh;
+  // lanes past the end of a partial last chunk compute the last site and drop it
+  const uint32_t e = active ? (uint32_t)(chunk * 64 + lane) : (uint32_t)(g.Vh - 1);
+  const Site s = site_of(g, op, e);
+  const void* ub = U.data[op];
+  const double* det = &U.det[op][0][0];
+  const R anis = (R)anis_d;
+  const bool ua = use_anis != 0;
+  if (w == 0) split_direction_to<SP, LK, R, 0, CP>(g, s, e, in, ub, det, U.unit, anis, ua, xch, lane);
+  else if (w == 1) split_direction_to<SP, LK, R, 1, CP>(g, s, e, in, ub, det, U.unit, anis, ua, xch, lane);
+  else if (w == 2) split_direction_to<SP, LK, R, 2, CP>(g, s, e, in, ub, det, U.unit, anis, ua, xch, lane);
+  else split_direction_to<SP, LK, R, 3, CP>(g, s, e, in, ub, det, U.unit, anis, ua, xch, lane);
+  __syncthreads();
+  if (w != 0) return;
+  double nrm = 0;
+  if (active) {
+    cx<R> o[12];
+#pragma unroll
+    for (int k = 0; k < 12; k++) o[k] = ((xch[0][k][lane] + xch[1][k][lane]) + xch[2][k][lane]) + xch[3][k][lane];
+    nrm = hop_epilogue<SP, MODE, XP, R, CLV, CP>(g, epi, out, e, 0, st, o);
+  }
+  if constexpr (MODE != 0) store_partial(nrm, partial, nchunks, 0, chunk);
+}
+
 // ---------------------------------------------------------------- register-blocked RHS
 // One slot of the hop for RB right-hand sides r0..r0+nrb-1 of the same site: the
 // link is loaded once and applied to each right-hand side's projected neighbour.
@@ -986,11 +1042,21 @@ inline bool links_stay(const Geo& g, int sp, int lk, const HopEpi& epi)
 // 9.1 / 9.7; 24^3x48, FP16 links 25.5 / 25.6.
 inline bool use_lds(int sp, bool keep) { return sp == SP_F64 || !keep; }
 
-// FP64 hops of one right-hand side split the directions over the wavefronts below 2^18
-// sites per parity, where the persistent kernel does not fill its slots twice.  Split
-// against one thread per site: 8^4 10.3 / 4.6 us, 12x6x10x14 14.5 / 4.7, 24x12^3 16.6 / 7.4,
-// 16^3x32 20.2 / 18.6, 20^3x40 55.0 / 48.6; above, 24^3x48 98 / 103, 28^3x56 177 / 190.
-inline bool use_split(const Geo& g) { return g.Vh < 1024 * kStageSites; }
+// Hops of one right-hand side split the directions over the wavefronts of a workgroup
+// (k_tm_hop_split and k_tm_hop_split_any) on lattices below a number of sites per parity.
+// Plain FP64 below 2^18, where the persistent kernel does not fill its slots twice; one
+// thread per site / split: hop on 8^4 10.3 / 4.6 us, 12x6x10x14 14.5 / 4.7, 24x12^3 16.6 /
+// 7.4, 16^3x32 20.2 / 18.6, 20^3x40 55.0 / 48.6; above, 24^3x48 98 / 103, 28^3x56 177 / 190.
+// The others finish a site in one wavefront of four and lose sooner.  Sloppy precisions
+// below 2^17: FP16 inner solves at 8^3x16 3.22 / 2.35 ms, 24x12^3 3.52 / 2.65, 16^3x32 4.42 /
+// 3.95 (FP32 4.49 / 4.31), 20^3x40 6.95 / 6.98.  Clover blocks, FP16 and FP32 below 2^15:
+// 24x12^3 3.89 / 3.06 ms, 16^3x32 4.92 / 5.21; FP64 below 2^13: 8^3x16 3.76 / 3.18 ms,
+// 24x12^3 4.67 / 5.20.
+inline bool use_split(const Geo& g, int sp, bool plain64, bool clover)
+{
+  const int bits = plain64 ? 18 : (!clover ? 17 : (sp == SP_F64 ? 13 : 15));
+  return g.Vh < (int64_t(1) << bits);
+}
 
 // Batched FP16 hops run k_tm_hop_rl, except one or two right-hand sides on a lattice that
 // fills the chip twice over with 256-site blocks: there the links of a site serve too few
@@ -1096,24 +1162,28 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
   const int ua = anis != 1.0 ? 1 : 0;
   const bool keep = links_stay(g, SP, LK, epi);
   const bool lds_ok = nr == 1 && L.s.W == 4 && !(lenv && lenv[0] == '0') && use_lds(SP, keep);
-  if constexpr (SP == SP_F64 && XP == SP_F64 && CLV == 0) {
-    if (nr == 1 && use_split(g) && !epi.coef && !(MODE == 3 && epi.rs.data)) {
-      HopEpi ks = epi;
-      fold_here = MODE == 0 && epi.fold_fin != FIN_NONE && epi.st;
-      if (!fold_here) ks.fold_fin = FIN_NONE;
-      const dim3 sg((unsigned)(L.nchunks + (fold_here ? 1 : 0)));
+  // the specialised FP64 kernel has no precision conversion and no clover blocks
+  constexpr bool plain64 = SP == SP_F64 && XP == SP_F64 && CLV == 0;
+  if (nr == 1 && !epi.coef && use_split(g, SP, plain64, CLV != 0)) {
+    HopEpi ks = epi;
+    fold_here = MODE == 0 && epi.fold_fin != FIN_NONE && epi.st;
+    if (!fold_here) ks.fold_fin = FIN_NONE;
+    const dim3 sg((unsigned)(L.nchunks + (fold_here ? 1 : 0)));
+    double* part = ctx->partial + epi.part0;
+    if constexpr (plain64) {
       if (keep)
-        NQ_HOP_LAUNCH((k_tm_hop_split<LK, MODE, 0>), sg, dim3(256), g, op, out, in, U, anis, ua, ks, L.nchunks,
-                      ctx->partial + epi.part0);
+        NQ_HOP_LAUNCH((k_tm_hop_split<LK, MODE, 0>), sg, dim3(256), g, op, out, in, U, anis, ua, ks, L.nchunks, part);
       else
-        NQ_HOP_LAUNCH((k_tm_hop_split<LK, MODE, kNT>), sg, dim3(256), g, op, out, in, U, anis, ua, ks, L.nchunks,
-                      ctx->partial + epi.part0);
-      prof_end_ext(ctx);
-      NQ_HIP(hipGetLastError());
-      if (epi.fold_fin != FIN_NONE && !fold_here) NQ_TRY(launch_finalize(ctx, 1, epi.st, epi.fold_fin, epi.fold_pred));
-      if (MODE != 0 && epi.fin != FIN_PARTIAL) NQ_TRY(launch_finalize(ctx, nr, epi.st, epi.fin, epi.pred_reliable));
-      return NQ_OK;
+        NQ_HOP_LAUNCH((k_tm_hop_split<LK, MODE, kNT>), sg, dim3(256), g, op, out, in, U, anis, ua, ks, L.nchunks, part);
+    } else {
+      NQ_HOP_LAUNCH((k_tm_hop_split_any<SP, LK, MODE, XP, CLV, 0>), sg, dim3(256), g, op, out, in, U, anis, ua, ks,
+                    L.nchunks, part);
     }
+    prof_end_ext(ctx);
+    NQ_HIP(hipGetLastError());
+    if (epi.fold_fin != FIN_NONE && !fold_here) NQ_TRY(launch_finalize(ctx, 1, epi.st, epi.fold_fin, epi.fold_pred));
+    if (MODE != 0 && epi.fin != FIN_PARTIAL) NQ_TRY(launch_finalize(ctx, nr, epi.st, epi.fin, epi.pred_reliable));
+    return NQ_OK;
   }
   if (lds_ok && launch_persistent<SP, LK, MODE, XP, CLV>(ctx, op, out, in, U, anis, epi, L)) {
     fold_here = false;
