@@ -957,81 +957,24 @@ static int launch_rb(nq_ctx* ctx, int RB, int op, const SpinorView& out, const S
   return NQ_OK;
 }
 
-// Autotuner of the right-hand sides per wavefront of the batched sloppy hop: on the
-// first batched launch of a (precision, batch size) it times the write-only kernel
-// (no solver state, output into a scratch buffer) with RB = 1, 2 and 4 right-hand
-// sides per wavefront on the caller's input and links, and keeps the fastest for
-// every mode of that precision and batch size.  All RB build the same per-RHS code
-// (one unrolled copy per right-hand side), so the choice never changes a result; the
-// one-RHS kernel (RB = 0 in launch_rb) is not a candidate: its FP16 code schedules
-// the same arithmetic differently and does not give the same bits.  NQ_TUNE=0 or an
-// open graph capture use RB = 2.
-template <int SP, int LK, int XP>
-static int tuned_rb(nq_ctx* ctx, int op, const SpinorView& in, const LinkView& U, double anis, const HopEpi& epi,
-                    int nr, int* rb)
-{
-  const std::string key = "tm_hop_rb/" + std::to_string(SP) + "/" + std::to_string(LK) + "/" + std::to_string(nr);
-  auto it = ctx->tuned.find(key);
-  if (it != ctx->tuned.end()) {
-    *rb = it->second;
-    return NQ_OK;
-  }
-  const char* env = getenv("NQ_TUNE");
-  if (ctx->capturing || (env && env[0] == '0')) {
-    *rb = 2;
-    return NQ_OK;
-  }
-  SpinorView scratch;
-  NQ_TRY(alloc_spinor_nr(ctx, "tune.out" + std::to_string(SP), SP, 12, nr, &scratch));
-  HopEpi e0;
-  e0.nrhs = nr;
-  e0.batched = 1;
-  e0.coef = epi.coef;
-  const bool prof = ctx->profiling;
-  ctx->profiling = false;
-  hipEvent_t a, b;
-  NQ_HIP(hipEventCreate(&a));
-  NQ_HIP(hipEventCreate(&b));
-  float best = 1e30f;
-  int best_rb = 2;
-  for (int cand : {1, 2, 4}) {
-    if (cand > 1 && cand > nr) continue;
-    NQ_TRY((launch_rb<SP, LK, 0, XP>(ctx, cand, op, scratch, in, U, anis, e0, nr)));  // warm-up
-    NQ_HIP(hipEventRecord(a, ctx->stream));
-    for (int i = 0; i < 3; i++) NQ_TRY((launch_rb<SP, LK, 0, XP>(ctx, cand, op, scratch, in, U, anis, e0, nr)));
-    NQ_HIP(hipEventRecord(b, ctx->stream));
-    NQ_HIP(hipEventSynchronize(b));
-    float ms = 0;
-    NQ_HIP(hipEventElapsedTime(&ms, a, b));
-    if (ms < best * 0.98f) {  // prefer the smaller block unless clearly slower
-      best = ms;
-      best_rb = cand;
-    }
-  }
-  (void)hipEventDestroy(a);
-  (void)hipEventDestroy(b);
-  ctx->profiling = prof;
-  ctx->tuned[key] = best_rb;
-  *rb = best_rb;
-  return NQ_OK;
-}
-
 // Whether the links and the data used once are accessed with the default cache policy,
 // to be found in the 256 MB memory-side cache by the next hop, instead of streamed past
 // it: when the links of both parities (and the clover blocks of K) and the input and
-// output spinors take at most 224 MB.  Measured, default against streamed, whole solves
+// output spinors take at most 224 MB (150 MB for several right-hand sides, whose other
+// vectors grow with them).  Measured, default against streamed, whole solves
 // (links of both parities): 123 MB (FP16 inner, 20^3x40) 7.41 against 8.23 ms, 127 MB
 // (FP16 links, 24^3x48) 11.6 / 12.7, 151 MB (FP64, 16^3x32) 7.56 / 8.03, 184 MB (FP32,
 // 20^3x40) 9.35 / 10.2; above it 236 MB (FP16 links, 28^3x56) 22.0 / 21.2, 255 MB (FP16
 // inner, 24^3x48) 14.5 / 14.1, 369 MB (FP64, 20^3x40) 19.9 / 19.0, 805 MB (FP16 inner,
 // 32^3x64) 41.2 / 37.4.  Twelve FP16 right-hand sides: 50 MB of links 21.8 / 22.1, 123 MB
-// (and 200 MB of spinors) 56.6 / 54.6, 255 MB 114.6 / 108.6.
+// (and 200 MB of spinors) 56.6 / 54.6, 255 MB 114.6 / 108.6; five at 46x16x22x20, 124 and
+// 84 MB, 26.4 / 25.9.
 inline bool links_stay(const Geo& g, int sp, int lk, const HopEpi& epi)
 {
   const int eb = sp == SP_F64 ? 16 : (sp == SP_F32 ? 8 : 4);
   double site = 2.0 * 8 * lk_nc(lk) * lk_eb(lk) + 2.0 * 12 * eb * epi.nrhs;
   if (epi.blk_mode) site += (72 + 36) * eb;
-  return site * (double)g.Vh <= 224.0 * 1048576;
+  return site * (double)g.Vh <= (epi.nrhs > 1 ? 150.0 : 224.0) * 1048576;
 }
 
 // Neighbours staged in LDS (k_tm_hop_lds) for one right-hand side: FP64 always (4 % at
@@ -1057,13 +1000,6 @@ inline bool use_split(const Geo& g, int sp, bool plain64, bool clover)
   const int bits = plain64 ? 18 : (!clover ? 17 : (sp == SP_F64 ? 13 : 15));
   return g.Vh < (int64_t(1) << bits);
 }
-
-// Batched FP16 hops run k_tm_hop_rl, except one or two right-hand sides on a lattice that
-// fills the chip twice over with 256-site blocks: there the links of a site serve too few
-// right-hand sides to pay for k_tm_hop_rl's two wavefronts per SIMD (32^3x64: one 100.5
-// against 116 us, two 150 against 157, three 208 against 190; 24^3x48: 31.7 / 33.7, 44.0 /
-// 46.2, 58.7 / 57.8; 16^3x32, 256 blocks: 12.6 / 10.1, 13.5 / 11.6).
-inline bool use_rl(int sp, const Geo& g, int nr) { return sp == SP_F16 && (nr > 2 || g.Vh < 1024 * kStageSites); }
 
 // launch of k_tm_hop_rl: the right-hand sides split into the fewest groups that give
 // every CU its two resident workgroups (16^3x32, 12 right-hand sides: one group 42.5 us,
@@ -1095,6 +1031,85 @@ static int launch_rl(nq_ctx* ctx, int op, const SpinorView& out, const SpinorVie
     (void)ctx; (void)op; (void)out; (void)in; (void)U; (void)anis; (void)epi; (void)nr;
     return fail(NQ_EINVAL, "tm hop: links in registers need FP16 spinors");
   }
+}
+
+// Autotuner of the right-hand sides per wavefront of the batched sloppy hop: on the
+// first batched launch of a (precision, batch size) it times the write-only kernel
+// (no solver state, output into a scratch buffer) with RB = 1, 2 and 4 right-hand
+// sides per wavefront on the caller's input and links, and keeps the fastest for
+// every mode of that precision and batch size.  FP16 has k_tm_hop_rl as a further
+// candidate (kTunedRl), which wins from three or four right-hand sides up and on small
+// lattices: 24^3x48, one right-hand side 31.7 us register-blocked / 33.7, two 44.0 / 46.2,
+// three 58.7 / 57.8, four 71 / 68, twelve 216 / 177; 32^3x64 100 / 116, 150 / 157, 208 /
+// 190, -, 682 / 517; 16^3x32 12.6 / 10.1, 13.5 / 11.6, 14.9 / 15.3, 17.5 / 18.7, 42 / 36.
+// It also loses where its 512 resident workgroups are filled a little more than once
+// (633 blocks, three right-hand sides).  All candidates build the same per-RHS code
+// (one unrolled copy per right-hand side), so the choice never changes a result; the
+// one-RHS kernel (RB = 0 in launch_rb) is not a candidate: its FP16 code schedules
+// the same arithmetic differently and does not give the same bits.  NQ_TUNE=0 or an
+// open graph capture use RB = 2, NQ_TUNE=r k_tm_hop_rl.
+constexpr int kTunedRl = 16;
+
+template <int SP, int LK, int MODE, int XP>
+static int launch_tuned(nq_ctx* ctx, int choice, int op, const SpinorView& out, const SpinorView& in,
+                        const LinkView& U, double anis, const HopEpi& epi, int nr)
+{
+  if (choice == kTunedRl) return launch_rl<SP, LK, MODE, XP>(ctx, op, out, in, U, anis, epi, nr);
+  return launch_rb<SP, LK, MODE, XP>(ctx, choice, op, out, in, U, anis, epi, nr);
+}
+
+template <int SP, int LK, int XP>
+static int tuned_rb(nq_ctx* ctx, int op, const SpinorView& in, const LinkView& U, double anis, const HopEpi& epi,
+                    int nr, int* rb)
+{
+  const std::string key = "tm_hop_rb/" + std::to_string(SP) + "/" + std::to_string(LK) + "/" + std::to_string(nr);
+  auto it = ctx->tuned.find(key);
+  if (it != ctx->tuned.end()) {
+    *rb = it->second;
+    return NQ_OK;
+  }
+  const char* env = getenv("NQ_TUNE");
+  if (ctx->capturing || (env && env[0] == '0')) {
+    *rb = 2;
+    return NQ_OK;
+  }
+  if (SP == SP_F16 && env && env[0] == 'r') {
+    *rb = kTunedRl;
+    return NQ_OK;
+  }
+  SpinorView scratch;
+  NQ_TRY(alloc_spinor_nr(ctx, "tune.out" + std::to_string(SP), SP, 12, nr, &scratch));
+  HopEpi e0;
+  e0.nrhs = nr;
+  e0.batched = 1;
+  e0.coef = epi.coef;
+  const bool prof = ctx->profiling;
+  ctx->profiling = false;
+  hipEvent_t a, b;
+  NQ_HIP(hipEventCreate(&a));
+  NQ_HIP(hipEventCreate(&b));
+  float best = 1e30f;
+  int best_rb = 2;
+  for (int cand : {1, 2, 4, kTunedRl}) {
+    if (cand == kTunedRl ? SP != SP_F16 : cand > nr) continue;
+    NQ_TRY((launch_tuned<SP, LK, 0, XP>(ctx, cand, op, scratch, in, U, anis, e0, nr)));  // warm-up
+    NQ_HIP(hipEventRecord(a, ctx->stream));
+    for (int i = 0; i < 3; i++) NQ_TRY((launch_tuned<SP, LK, 0, XP>(ctx, cand, op, scratch, in, U, anis, e0, nr)));
+    NQ_HIP(hipEventRecord(b, ctx->stream));
+    NQ_HIP(hipEventSynchronize(b));
+    float ms = 0;
+    NQ_HIP(hipEventElapsedTime(&ms, a, b));
+    if (ms < best * 0.98f) {  // prefer the smaller block unless clearly slower
+      best = ms;
+      best_rb = cand;
+    }
+  }
+  (void)hipEventDestroy(a);
+  (void)hipEventDestroy(b);
+  ctx->profiling = prof;
+  ctx->tuned[key] = best_rb;
+  *rb = best_rb;
+  return NQ_OK;
 }
 
 // Launches the persistent staged hop and returns true when it applies: FP64
@@ -1137,12 +1152,10 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
       // sides per wavefront, chosen by the autotuner for this precision and batch.
       // FP64 too: the reliable updates of a batch share each link load (measured
       // 953 -> 879 us for 12 sources, the batched FP64 solve 95 -> 85 ms per source)
-      const bool rl = use_rl(SP, g, nr);
       int RB = 0;
-      if (!rl) NQ_TRY((tuned_rb<SP, LK, XP>(ctx, op, in, U, anis, epi, nr, &RB)));
+      NQ_TRY((tuned_rb<SP, LK, XP>(ctx, op, in, U, anis, epi, nr, &RB)));
       prof_begin_ext(ctx, name, tm_hop_bytes(SP, LK, epi) * (double)g.Vh, &ctx->hop_ev[0], &ctx->hop_ev[1]);
-      const int rc = rl ? launch_rl<SP, LK, MODE, XP>(ctx, op, out, in, U, anis, epi, nr)
-                        : launch_rb<SP, LK, MODE, XP>(ctx, RB, op, out, in, U, anis, epi, nr);
+      const int rc = launch_tuned<SP, LK, MODE, XP>(ctx, RB, op, out, in, U, anis, epi, nr);
       prof_end_ext(ctx);
       NQ_TRY(rc);
       if (epi.fold_fin != FIN_NONE) NQ_TRY(launch_finalize(ctx, nr, epi.st, epi.fold_fin, epi.fold_pred));

@@ -1,8 +1,8 @@
 """Variants of the twisted-mass hop kernels at the sizes where their dispatch changes.
 
 * The batched FP16 hop keeps the links of a site in registers and loops over its
-  right-hand sides, in one or several groups; one or two right-hand sides on a large
-  lattice run the register-blocked kernel instead.  A source has the same bits alone and
+  right-hand sides, in one or several groups; the tuner may take the register-blocked
+  kernel instead.  A source has the same bits alone and
   in a batch whichever kernel and grouping the batch size picks, and small lattices agree
   with the oracle (1e-10, the bar of the other mixed solves at residue 1e-24).
 * Links with a phase in every direction (the det of each slot enters the third row) and
@@ -25,8 +25,7 @@ def conf_of(L, seed, theta):
     return conf
 
 
-# the largest has 262144 sites per parity, where one right-hand side runs another kernel
-# than three; 16^3x32 splits five right-hand sides into two groups
+# 16^3x32 splits five right-hand sides into two groups
 @pytest.mark.parametrize("L,nr", [((32, 16, 16, 16), 5), ((16, 32, 32, 32), 3)])
 @pytest.mark.parametrize("prec", ["f16", "f16h"])
 def test_batched_f16_same_bits_alone(L, nr, prec):
@@ -42,6 +41,26 @@ def test_batched_f16_same_bits_alone(L, nr, prec):
             one = [ctx.field(nq.SPINCOLOR, nq.LX)]
             nq.tm_solve_eoprec_multi(ctx, g, 0.16, mus[i:i + 1], 1000, 1e-14, one, src[i:i + 1], prec=prec)
             assert np.array_equal(one[0].download(), sol[i].download()), i
+
+
+# the register-blocked kernel (NQ_TUNE=0) and the one with the links in registers
+# (NQ_TUNE=r), whichever the tuner would take: every epilogue of a solve, same bits
+@pytest.mark.parametrize("L,nr", [((10, 4, 2, 2), 3), ((32, 16, 16, 16), 5), ((46, 16, 22, 20), 2)])
+@pytest.mark.parametrize("prec", ["f16", "f16h"])
+def test_batched_f16_kernels_agree(L, nr, prec, monkeypatch):
+    conf = conf_of(L, 55, [1.0, 0.2, 0, 0])
+    sols = []
+    for tune in ("0", "r"):
+        monkeypatch.setenv("NQ_TUNE", tune)
+        with nq.Ctx(L) as ctx:
+            g = nq.Gauge(ctx, lx=conf)
+            src = [ctx.field(nq.SPINCOLOR, nq.LX, nq.source_lx(L, 90 + i)) for i in range(nr)]
+            sol = [ctx.field(nq.SPINCOLOR, nq.LX) for _ in range(nr)]
+            res = nq.tm_solve_eoprec_multi(ctx, g, 0.16, [0.05] * nr, 1000, 1e-14, sol, src, prec=prec)
+            assert all(r["rc"] == nq.NQ_OK for r in res), res
+            sols.append([f.download() for f in sol])
+    for i in range(nr):
+        assert np.array_equal(sols[0][i], sols[1][i]), i
 
 
 @pytest.mark.parametrize("L", [(10, 4, 2, 2), (4, 6, 4, 10), (8, 4, 4, 12)])
