@@ -360,7 +360,8 @@ __global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop(Geo g, i
 
 // The accumulators are pinned after every slot for FP16 (76-87 registers instead of 128,
 // five or six wavefronts per SIMD beside the 13 KB of LDS: 32^3x64 hop 88 -> 85 us, FP16
-// links 74 -> 61), after every four slots otherwise (FP32 139 -> 132 us).
+// links 74 -> 61), after every two for FP64 with 12-real links (FP16 solve at 32^3x64
+// 36.05 -> 35.73 ms), after every four otherwise (FP32 139 -> 132 us).
 // One right-hand side, neighbours staged in LDS (Stage): the workgroup's four
 // wavefronts cover 256 consecutive output sites (Shape W = 4, NRB = 1).
 template <int SP, int LK, int MODE, int XP, int CLV = 0, int CP = kNT>
@@ -396,7 +397,7 @@ __global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop_lds(Geo 
     cx<R> o[12];
 #pragma unroll
     for (int k = 0; k < 12; k++) o[k] = mk<R>(0, 0);
-    hop_site<SP, LK, R, SP == SP_F16 ? 1 : 4, CP, true>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
+    hop_site<SP, LK, R, SP == SP_F16 ? 1 : (LK == LK_F64_12 ? 2 : 4), CP, true>(g, s, e, in, r, ub, det, unit, anis, ua, o, lds, e0);
     nrm = hop_epilogue<SP, MODE, XP, R, CLV, CP>(g, epi, out, e, r, st, o);
   }
   if constexpr (MODE != 0) store_partial(nrm, partial, nchunks, m.r, m.chunk);
