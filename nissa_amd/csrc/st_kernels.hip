@@ -811,14 +811,24 @@ static double lbytes(int lk) { return lk == LK_F64_18 ? 144.0 : 72.0; }
 // multi-shift hop 1214 against 1245 us with RB = 4; the 16-system refinement CG's
 // fused tail 511 against 534-557 us with RB = 8 or 4); else 4 (FP64: RB = 6 takes
 // 208 VGPRs and 72 KB of LDS, two wavefronts per SIMD, and measured 2 % slower).
+// A lattice with too few 256-site blocks for two workgroups per CU takes fewer per
+// wavefront, for more workgroups.  Multi-shift CG with the block above -> with the one
+// the rule takes: 16^3x32, 4 sources, 10 shifts, FP32 51.5 -> 46.9 ms, FP64 42.6 -> 39.1
+// (RB = 1: 58.1, 51.0); 26x14^3, 3 x 9, FP32 35.6 -> 30.5; 16x8^3, 4 x 12, 33.1 -> 24.4;
+// 20x10^3, 2 x 8, FP64 17.2 -> 14.5.  20^3x40, 4 x 10, FP64 keeps 4: 102.5 (2: 101.1,
+// 1: 126.5).
 // NQ_ST_RB = 1, 2, 4, 6 or 8 (8: FP32 only) overrides; every choice gives the same
 // bits.  The launch shape for RB: W = 4 chunks per workgroup, one RB group per
 // wavefront.
-static int st_rb(int nr, int sp)
+static int st_rb(const nq_ctx* ctx, int nr, int sp)
 {
   if (nr <= 1) return 1;
   const char* e = getenv("NQ_ST_RB");
-  const int v = e ? atoi(e) : (sp == SP_F32 && nr >= 5 ? 6 : 4);
+  int v = e ? atoi(e) : (sp == SP_F32 && nr >= 5 ? 6 : 4);
+  if (!e) {
+    const int64_t nblk = (ctx->geo.Vh + kStageSites - 1) / kStageSites;
+    while (v > 1 && nblk * ((nr + v - 1) / v) < 2 * ctx->ncu) v = v > 4 ? 4 : v / 2;
+  }
   if (v == 8) return sp == SP_F32 ? 8 : 4;
   return v == 1 || v == 2 || v == 6 ? v : 4;
 }
@@ -875,7 +885,7 @@ int launch_st_hop(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& 
   // links once for all right-hand sides, the fields per right-hand side
   const double by = 8 * lbytes(lk) + csite(sp) * (1 + (aux.data ? 1 : 0) + ((mode == 0 || write) ? 1 : 0)) * nr;
   prof_begin(ctx, mode == 0 ? "st_hop" : "st_hop_red", by * (double)g.Vh, &ev);
-  const int RB = st_rb(nr, sp);
+  const int RB = st_rb(ctx, nr, sp);
 #define NQ_ST(SPV, LKV)                                                                                              \
   switch (mode) {                                                                                                    \
   case 0: st_hop_go<SPV, LKV, 0>(ctx, RB, op, out, in, U, c1, c2, coef_dev, aux, write, nr, skip_flags, skip_stride, \
@@ -910,7 +920,7 @@ int launch_st_cgtail(nq_ctx* ctx, const SpinorView& t, const LinkView& U, const 
   hipEvent_t ev = nullptr;
   // links once; per system t gathered, p read, x and r read and written
   prof_begin(ctx, "st_cgtail", (8 * lbytes(lk) + 6 * csite(sp) * nr) * (double)g.Vh, &ev);
-  const int RB = st_rb(nr, sp);
+  const int RB = st_rb(ctx, nr, sp);
   const Shape sh = st_shape(nr, RB);
   const dim3 grid((unsigned)((nchunks + 3) / 4 * sh.NRG)), blk(256);
 #define NQ_TL(SPV, LKV, RBV)                                                                                        \
@@ -1109,7 +1119,7 @@ int launch_cgm_persistent(nq_ctx* ctx, const LinkView& U, const SpinorView& p, c
   A.none.ncomp = 3;
   A.sstride = sstride;
   A.nchunks = (g.Vh + 63) / 64;
-  const int RB = st_rb(nr, sp);
+  const int RB = st_rb(ctx, nr, sp);
   A.sh_hop = st_shape(nr, RB);
   A.blocks_hop = (A.nchunks + 3) / 4 * A.sh_hop.NRG;
   const Launch L = launch_shape(g, nr);
@@ -1168,7 +1178,7 @@ int launch_cgm_iteration(nq_ctx* ctx, const LinkView& U, const SpinorView& p, co
   // runs only before a reliable update)
   const double cs = csite(sp);
   prof_begin(ctx, "cgm_hop1", (8 * lbytes(lk) + 2 * cs * nbusy) * (double)g.Vh, &ev);
-  const int RB = st_rb(nr, sp);
+  const int RB = st_rb(ctx, nr, sp);
   const int* skip = (const int*)&st->done;
   const int sstr = (int)(sizeof(CgmState) / sizeof(int));
   if (sp == SP_F64)

@@ -7,13 +7,14 @@
   with the oracle (1e-10, the bar of the other mixed solves at residue 1e-24).
 * Links with a phase in every direction (the det of each slot enters the third row) and
   with a phase in t alone (it is left out elsewhere).
+* The staggered batch: same bits however many sources a wavefront takes.
 * Site orders whose z tile does not fit the extent (2 mod 4) or spans it.
 """
 import numpy as np
 import pytest
 
 import nissa_amd as nq
-from helpers import gauss_eo, rel_l2
+from helpers import gauss_eo, rel_l2, st_conf
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -127,3 +128,23 @@ def test_persistent_hop_same_bits_large(monkeypatch):
             assert st["rc"] == nq.NQ_OK
             out.append((fo.download(), fx.download()))
         assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+# fewer sources per wavefront on lattices of few blocks: 256, 128 and 18 blocks, one partial
+@pytest.mark.parametrize("L,nr", [((32, 16, 16, 16), 4), ((16, 16, 16, 16), 4), ((14, 10, 8, 8), 7), ((2, 4, 6, 2), 2)])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_staggered_batch_same_bits_whatever_the_block(L, nr, prec, monkeypatch):
+    out = {}
+    for rb in (None, "1", "4", "6"):
+        monkeypatch.delenv("NQ_ST_RB", raising=False)
+        if rb:
+            monkeypatch.setenv("NQ_ST_RB", rb)
+        with nq.Ctx(L) as ctx:
+            g = nq.Gauge(ctx, lx=st_conf(L, 7))
+            src = [ctx.field(nq.COLOR, nq.EVEN, gauss_eo(np.prod(L) // 2, 70 + i, ncomp=3)) for i in range(nr)]
+            sol = [[ctx.field(nq.COLOR, nq.EVEN) for _ in range(2)] for _ in src]
+            res = nq.st_cgm(ctx, g, [0.09, 0.5], 2000, [1e-16, 1e-16], sol, src, prec=prec)
+            assert all(r["rc"] == nq.NQ_OK for r in res), res
+            out[rb] = np.stack([f.download() for s in sol for f in s])
+    for rb in ("1", "4", "6"):
+        assert np.array_equal(out[None], out[rb]), rb
