@@ -323,7 +323,11 @@ __device__ __forceinline__ bool fold_finalise(const HopEpi& epi, const double* p
 }
 
 // workgroups of at most 256 threads; FP64 builds get the full 256-VGPR budget
-// (one wavefront per SIMD per workgroup), the sloppy builds two workgroups per CU
+// (one wavefront per SIMD per workgroup), the sloppy builds two workgroups per CU.
+// FP16 pins the accumulators after every slot: the registers it saves put all of a
+// middle lattice's wavefronts on the SIMDs at once.  FP16 links at 24^3x48 26.5 -> 24.1 us
+// and 20^3x40 14.4 -> 13.6, FP32 links 16.3 -> 15.1 (solves 11.5 -> 11.2, 6.57 -> 6.33,
+// 7.00 -> 6.86 ms), 16^3x32 equal; pins for FP32 are equal, four slots stay.
 template <int SP, int LK, int MODE, int XP, int CLV = 0, int CP = kNT>
 __global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop(Geo g, int op, SpinorView out, SpinorView in, LinkView U, double anis_d,
                                                int use_anis, HopEpi epi, Shape S, int64_t nchunks,
@@ -352,7 +356,7 @@ __global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop(Geo g, i
     cx<R> o[12];
 #pragma unroll
     for (int k = 0; k < 12; k++) o[k] = mk<R>(0, 0);
-    hop_site<SP, LK, R, 4, CP, false>(g, s, e, in, r, ub, det, unit, anis, ua, o);
+    hop_site<SP, LK, R, SP == SP_F16 ? 1 : 4, CP, false>(g, s, e, in, r, ub, det, unit, anis, ua, o);
     nrm = hop_epilogue<SP, MODE, XP, R, CLV, CP>(g, epi, out, e, r, st, o);
   }
   if constexpr (MODE != 0) store_partial(nrm, partial, nchunks, m.r, m.chunk);
@@ -980,10 +984,10 @@ inline bool links_stay(const Geo& g, int sp, int lk, const HopEpi& epi)
 
 // Neighbours staged in LDS (k_tm_hop_lds) for one right-hand side: FP64 always (4 % at
 // 32^3x64), the sloppy precisions when the links are streamed: unstaged against staged,
-// FP32 54.4 / 49.8 us at 24^3x48 and 139 / 132 at 32^3x64; FP16 34.6 / 33.4 and 91 / 85;
-// FP16 links at 32^3x64 74.8 / 61.3.  With the links in the memory-side cache the staging
+// FP32 54.4 / 49.8 us at 24^3x48 and 139 / 132 at 32^3x64; FP16 34.1 / 33.4 and 91 / 86;
+// FP16 links at 32^3x64 66.5 / 63.5.  With the links in the memory-side cache the staging
 // round trip is not paid back: 16^3x32 FP32 10.7 / 12.0 us, FP16 9.4 / 10.1, FP16 links
-// 9.1 / 9.7; 24^3x48, FP16 links 25.5 / 25.6.
+// 9.1 / 9.7; 24^3x48, FP16 links 24.1 / 25.6.
 inline bool use_lds(int sp, bool keep) { return sp == SP_F64 || !keep; }
 
 // Hops of one right-hand side split the directions over the wavefronts of a workgroup
