@@ -315,7 +315,18 @@ __global__ void __launch_bounds__(256) k_st_cgtail(Geo g, SpinorView t, LinkView
 // C2: s = -1/4 Deo t (even output, never stored) ; sol_k -= betas_k ps_k ; r += betaa s ; |r|^2
 // sol/ps of shift k of rhs r: base + r*rstride + k*sstride (elements)
 // (RB right-hand sides per wavefront as in k_st_hop)
-template <int SP, int LK, int RB>
+// PERS: inside the persistent kernel, where the states change between phases of one launch;
+// else they are constant and come through scalar loads (a vector load behind the shift
+// vectors' loads and stores waits for all of them).  12 poles, 4 sources at 24^3x48 FP32
+// 221.1 -> 216.2 ms, 10 poles at 16^3x32 47.1 -> 45.8, 2 x 8 at 20x10^3 FP64 14.6 -> 13.9.
+template <bool PERS, class T>
+__device__ __forceinline__ T cst(const T* p)
+{
+  if constexpr (PERS) return *p;
+  else return sload(p);
+}
+
+template <int SP, int LK, int RB, bool PERS = false>
 __device__ __forceinline__ void cgm_hop2_block(int64_t lb, char* lds, const Geo& g, const SpinorView& t,
                                                const LinkView& U, const SpinorView& rv, const SpinorView& sol,
                                                const SpinorView& ps, int64_t sstride, const CgmState* st,
@@ -341,26 +352,26 @@ __device__ __forceinline__ void cgm_hop2_block(int64_t lb, char* lds, const Geo&
   for (int b = 0; b < RB; b++) {
     if (b >= nrb) continue;
     const int r = r0 + b;
-    const CgmState* S = st + r;
+    const CgmState* S = st + __builtin_amdgcn_readfirstlane(r);
     double red = 0;
     if (m.active && ((busy >> b) & 1u)) {
-      const R betaa = (R)S->betaa;
+      const R betaa = (R)cst<PERS>(&S->betaa);
       cx<R> rr[3];
       SpAcc<SP, R, 3, kNT>::load(rv, g.stride, m.e, rr, r);
-      const bool pend = S->pend != 0;
+      const bool pend = cst<PERS>(&S->pend) != 0;
       // lag: the last hop2 left its terms betas_prev_k ps_k(previous) to this one
       // (then pend is set too, so the stored ps_k is still the previous iteration's)
-      const bool lag = S->lag != 0;
+      const bool lag = cst<PERS>(&S->lag) != 0;
       // shifts in groups of G, every load of a group issued before its first store
       // (one memory wait per group instead of one per shift)
       constexpr int G = SP == SP_F64 ? 2 : 4;
       const int64_t kb = sstride * (SP == SP_F64 ? 16 : 8);  // bytes between shifts
-      for (int k0 = 0; k0 < S->nshift; k0 += G) {
+      for (int k0 = 0; k0 < cst<PERS>(&S->nshift); k0 += G) {
         bool on[G];
         bool any = false;
 #pragma unroll
         for (int j = 0; j < G; j++) {
-          on[j] = k0 + j < S->nshift && S->run[k0 + j];
+          on[j] = k0 + j < cst<PERS>(&S->nshift) && cst<PERS>(&S->run[k0 + j]);
           any = any || on[j];
         }
         if (!any) continue;  // uniform over the wavefront
@@ -390,7 +401,7 @@ __device__ __forceinline__ void cgm_hop2_block(int64_t lb, char* lds, const Geo&
           if (pend) {
             // the last iteration's C3 update ps_k = zeta_k r + alpha_k ps_k (r not yet
             // updated; zas_k holds the zfs_k that C3 would use, alphas_k is unchanged)
-            const R z = (R)S->zas[k], al = (R)S->alphas[k];
+            const R z = (R)cst<PERS>(&S->zas[k]), al = (R)cst<PERS>(&S->alphas[k]);
 #pragma unroll
             for (int c = 0; c < 3; c++) {
               q[j][c].re = fma(al, q[j][c].re, z * rr[c].re);
@@ -403,7 +414,7 @@ __device__ __forceinline__ void cgm_hop2_block(int64_t lb, char* lds, const Geo&
           if (!lag) continue;  // this iteration's term waits for the next hop2
           // sol_k -= betas_prev_k ps_k(previous) ; sol_k -= betas_k ps_k, in that
           // order: the bits of two separate updates
-          const R bp = (R)S->betas_prev[k], bk = (R)S->betas[k];
+          const R bp = (R)cst<PERS>(&S->betas_prev[k]), bk = (R)cst<PERS>(&S->betas[k]);
 #pragma unroll
           for (int c = 0; c < 3; c++) {
             x[j][c].re = fma(-bp, qo[j][c].re, x[j][c].re);
@@ -739,7 +750,7 @@ __global__ void __launch_bounds__(256) k_cgm_persistent(CgmPArgs A)
     // C2: hop + shift and r updates, |r|^2 partials
     for (int64_t lb = f; lb < hi; lb += step) {
       __syncthreads();
-      cgm_hop2_block<SP, LK, RB>(lb, lds, A.g, A.t, A.U, A.r, A.sol, A.ps, A.sstride, A.st, A.sh_hop, A.nr,
+      cgm_hop2_block<SP, LK, RB, true>(lb, lds, A.g, A.t, A.U, A.r, A.sol, A.ps, A.sstride, A.st, A.sh_hop, A.nr,
                                  A.nchunks, A.partial);
     }
     if (!grid_sync(A.bar, &gen, A.spin_limit, &s_ok)) return;
