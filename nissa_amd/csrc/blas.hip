@@ -146,6 +146,20 @@ __device__ __forceinline__ bool rr_inline(const BlasArgs& A, double* vl, double*
   return !(isnan(tot) || sqrt(tot) < s->delta * s->r0 || tot < s->target || last);
 }
 
+// Whether the p update of right-hand side m.r idles.  A stop that a finalisation riding in a
+// hop left (CgState::stop) becomes done / reliable here: with it set, no workgroup of this
+// launch reads those two.
+__device__ __forceinline__ bool pupdate_idle(const BlasArgs& A, const Map& m)
+{
+  CgState* s = A.st + m.r;
+  const int stop = s->stop;
+  if (stop) {
+    if (m.chunk == 0 && (threadIdx.x & 63) == 0) raise_stop<false>(s, stop);
+    return true;
+  }
+  return s->done || (A.pred == 2 ? !s->reliable : s->reliable);
+}
+
 // p = r + beta p, beta from state[r]; skipped once that right-hand side is done or
 // while it waits for a reliable update.  With x given, first x += alpha p (the CG
 // solution update moved out of the matvec tail, so that p is read once per
@@ -155,7 +169,7 @@ __global__ void __launch_bounds__(256) k_pupdate(BlasArgs A, SpinorView p, Spino
 {
   const Map m = map_thread(A.s, A.g.Vh);
   const CgState* s = A.st + m.r;
-  if (s->done || (A.pred == 2 ? !s->reliable : s->reliable)) return;  // uniform per right-hand side
+  if (pupdate_idle(A, m)) return;  // uniform per right-hand side
   double beta;
   if (A.fin != FIN_NONE) {
     __shared__ double vl[1024];
@@ -197,7 +211,7 @@ __global__ void __launch_bounds__(256) k_pupdate_pair(BlasArgs A, SpinorView pin
 {
   const Map m = map_thread(A.s, A.g.Vh);
   const CgState* s = A.st + m.r;
-  if (s->done || s->reliable) return;
+  if (pupdate_idle(A, m)) return;
   double beta;
   bool xstep;
   if (A.fin != FIN_NONE) {
@@ -314,7 +328,7 @@ __global__ void __launch_bounds__(1024) k_finalize(const double* partial, int64_
   __shared__ double vl[1024];
   CgState* s = st + blockIdx.x;
   // uniform over the workgroup
-  if (s->done || (pred_reliable == 1 && !s->reliable) || (pred_reliable == 2 && s->reliable)) return;
+  if (s->stop || s->done || (pred_reliable == 1 && !s->reliable) || (pred_reliable == 2 && s->reliable)) return;
   const double tot = block_sum_partials(partial + (int64_t)blockIdx.x * nchunks, nchunks, vl);
   if (threadIdx.x == 0) finalize(s, fin, tot);
 }
@@ -466,6 +480,8 @@ int launch_cg_pupdate(nq_ctx* ctx, const SpinorView& p, const SpinorView& r, CgS
 
 __global__ void k_cg_commit(CgState* st)
 {
+  raise_stop<false>(st, st->stop);
+  st->stop = 0;
   if (!st->pending) return;
   const int f = st->pending;
   st->pending = FIN_NONE;

@@ -486,87 +486,6 @@ __device__ __forceinline__ double wave_sum(double v)
   return v;
 }
 
-// One recurrence of the CG / mixed CG.  FIN_PAP first records a finalisation that the p
-// update left pending; when that one stops the source or raises `reliable`, alpha stays.
-__device__ inline void finalize(CgState* st, int fin, double total)
-{
-  if (fin == FIN_PAP && st->pending) {
-    const int f = st->pending;
-    st->pending = FIN_NONE;
-    finalize(st, f, st->rr_new);
-    if (st->done || st->reliable) return;
-  }
-  switch (fin) {
-  case FIN_STORE0: st->extra[0] = total; break;
-  case FIN_STORE1: st->extra[1] = total; break;
-  case FIN_PAP:
-    st->pAp = total;
-    st->alpha_prev = st->alpha;
-    st->alpha = st->rr / total;
-    if (!(total > 0.0) || isnan(total)) { st->nan = 1; st->done = 1; }
-    break;
-  case FIN_RR: {
-    const double rr_new = total;
-    st->iter += 1;
-    st->beta = rr_new / st->rr;
-    st->rr = rr_new;
-    if (isnan(st->beta)) { st->nan = 1; st->done = 1; }
-    if (!(rr_new >= st->target) || st->iter >= st->niter) st->done = 1;
-    break;
-  }
-  case FIN_RR_SLOPPY: {
-    // mixed CG: when |r| has dropped by delta since the last FP64 residual (or the
-    // sloppy residual reached the target, or the iteration budget is spent) raise
-    // `reliable`: the sloppy kernels then idle until the host has run the FP64
-    // reliable update, whose finalisation (FIN_RR_TRUE) clears it again.
-    const double rr_new = total;
-    st->iter += 1;
-    st->rr_new = rr_new;
-    if (isnan(rr_new)) { st->nan = 1; st->done = 1; break; }
-    if (sqrt(rr_new) < st->delta * st->r0 || rr_new < st->target || st->iter >= st->niter) {
-      st->reliable = 1;
-    } else {
-      st->beta = rr_new / st->rr;
-      st->rr = rr_new;
-      // paired x updates: this p update applies two terms when the last one left its own
-      st->xstep = st->xlag;
-      st->xlag = !st->xlag;
-    }
-    break;
-  }
-  case FIN_RR_TRUE:
-  case FIN_RR_TRUE_HOLD: {
-    const double rr_true = total;
-    st->nreliable += 1;
-    st->true_rr = rr_true;
-    st->beta = rr_true / st->rr;
-    st->rr = rr_true;
-    st->r0 = sqrt(rr_true);
-    st->xlag = 0;  // the reliable update has taken every x term
-    if (fin == FIN_RR_TRUE) st->reliable = 0;
-    if (isnan(rr_true)) { st->nan = 1; st->done = 1; }
-    if (rr_true < st->target || st->iter >= st->niter) st->done = 1;
-    break;
-  }
-  case FIN_INIT_B2:
-    st->b2 = total;
-    st->target *= total;
-    st->rr = total;
-    st->r0 = sqrt(total);
-    st->true_rr = total;
-    if (!(total > 0.0) || isnan(total)) { st->nan = 1; st->done = 1; }
-    break;
-  case FIN_RR_INIT:
-    st->rr = total;
-    st->r0 = sqrt(total);
-    st->true_rr = total;
-    if (isnan(total)) { st->nan = 1; st->done = 1; }
-    if (!(total >= st->target)) st->done = 1;
-    break;
-  default: break;
-  }
-}
-
 // Thread mapping shared by all field kernels: a block covers W chunks of 64
 // consecutive sites for NRB right-hand sides of group g (Shape); wavefront w
 // handles right-hand side g*NRB + w % NRB of chunk w / NRB.  Launch: 64*W*NRB

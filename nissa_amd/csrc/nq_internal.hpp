@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/nissa_amd.h"
+#include "cg_state.hpp"
 
 namespace nq {
 
@@ -88,74 +89,6 @@ struct LinkView {
   // bit mu: |det(U_mu) - 1| < 1e-13, the links of direction mu carry no phase.  The FP32
   // and FP16 link kernels then leave out the product with det, which is 1 in FP32
   unsigned unit = 0;
-};
-
-// Solver state living in device memory; updated by the finalisation kernel
-// that follows each reducing launch.
-struct CgState {
-  double b2, target;
-  double rr, rr_new, pAp, alpha, beta;
-  double r0, delta;     // reliable-update reference |r| and threshold factor
-  double true_rr;       // last FP64 residual
-  double extra[6];
-  double alpha_prev;    // alpha of the previous iteration (paired x updates)
-  // pending: a finalisation (Fin) of rr_new that the p update has acted on (launch_cg_pupdate
-  // with fin) and that the next FIN_PAP finalisation or launch_cg_commit records
-  int iter, niter, done, reliable, nreliable, nan, mixed, pending;
-  // paired x updates of the one-source mixed CG: xlag = the last p update left its
-  // alpha p term to the next one; xstep = the coming p update applies both terms
-  int xlag, xstep;
-};
-
-constexpr int kMaxShift = 16;
-
-// Multi-shift CG state of one source (cgm_invert recurrences); lives in device
-// memory, updated by the CGM finalisation kernels.
-// Mixed precision (mixed = 1): the sloppy solutions are flushed into FP64 and the
-// Krylov residual is replaced by the FP64 residual of the hardest running shift
-// (kref, the smallest running shift) whenever that shift's squared residual has
-// dropped by delta2 since the last such update.  reliable = 1: flagged at the end of an iteration
-// whose p/ps update still runs; 2: idle until the host's update clears it.
-struct CgmState {
-  double b2, rr, betaa, betap, alpha, rfrf, pap, rel_ref, delta2, pad0;
-  double shift[kMaxShift], target[kMaxShift], zps[kMaxShift], zas[kMaxShift], zfs[kMaxShift];
-  double betas[kMaxShift], alphas[kMaxShift], res[kMaxShift];
-  double betas_prev[kMaxShift];  // betas_k of the previous iteration (paired sol_k updates)
-  int run[kMaxShift];
-  // owe_k: the sol_k term betas_k ps_k of the last hop2 is still to be applied,
-  // 1 by the host's settle kernel (the shift stopped or the source ended), 2 by
-  // the update kernel (a reliable update follows)
-  int owe[kMaxShift];
-  int done, reliable;  // adjacent: the sloppy kernels skip a source when either is set
-  int nshift, nrun, iter, niter, nan, mixed, kref, nreliable;
-  // lx solves (launch_cgm_vec): the shift vectors are updated every other iteration, from
-  // the pending iteration's coefficients (b1, z1, a1; ran1: shifts that ran in it; ran2:
-  // in the current one).  vmode, set by the rfrf finalisation, is the next vector
-  // update's work: 0 none (idle after the end), 1 p only, keeping r (this iteration stays
-  // pending), 2 p and both iterations, 3 the last iteration alone (the end came on one)
-  double b1[kMaxShift], z1[kMaxShift], a1[kMaxShift];
-  int ran1[kMaxShift], ran2[kMaxShift];
-  int lx, vlag, vmode, pad1;
-  // pend: the ps_k update of the iteration just finalised is left to the next
-  // iteration's hop2 kernel (set by the rfrf finalisation when the source goes on
-  // without a reliable update; the update kernel then updates p only)
-  // lag: the last hop2 left its sol_k terms to the next one, which applies both
-  // iterations' terms in order (so sol_k is read and written every other iteration)
-  int pend, lag;
-};
-
-enum Fin {
-  FIN_NONE = 0,
-  FIN_STORE0 = 1,     // extra[0] = total
-  FIN_PAP = 2,        // pAp = total; alpha = rr/pAp
-  FIN_RR = 3,         // plain CG: beta, rr, iter, done
-  FIN_RR_SLOPPY = 4,  // mixed CG: decide reliable update
-  FIN_RR_TRUE = 5,    // mixed CG: after FP64 recomputation
-  FIN_RR_INIT = 6,    // initial residual: rr = total, r0 = sqrt
-  FIN_STORE1 = 7,     // extra[1] = total
-  FIN_RR_TRUE_HOLD = 8,  // as FIN_RR_TRUE, but `reliable` stays raised (batched updates)
-  FIN_INIT_B2 = 9,    // start of a solve on r = b: b2 = rr = total, target *= total
-  FIN_PARTIAL = 10,   // leave the per-chunk partials for a caller's own finalisation
 };
 
 // Hop epilogue: out_h = c1_h*hop + c2_h*aux + c3_h*aux2 (h = upper/lower spins).

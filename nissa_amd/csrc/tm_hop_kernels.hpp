@@ -302,14 +302,20 @@ __device__ __forceinline__ double hop_epilogue(const Geo& g, const HopEpi& epi, 
   return nrm;
 }
 
+// Whether the launch skips a right-hand side.  done and reliable are constant over the
+// launch: a finalisation that rides in it (fold_finalise, mode 0) leaves its own to `stop`,
+// which the CG tail right after it (mode 2) reads as well.
+template <int MODE>
 __device__ __forceinline__ bool rhs_idle(const CgState* st, int pred)
 {
   const int reliable = sload(&st->reliable);
-  return sload(&st->done) || (pred == 1 && !reliable) || (pred == 2 && reliable);
+  const int done = sload(&st->done) | (MODE == 2 ? sload(&st->stop) : 0);
+  return done || (pred == 1 && !reliable) || (pred == 2 && reliable);
 }
 
 // The workgroup past the last block finalises the previous launch's reduction (one
-// right-hand side; the hop itself never reads what it writes); vl: 1024 doubles of LDS.
+// right-hand side); vl: 1024 doubles of LDS.  It writes nothing that the hop reads: the
+// wavefronts of a workgroup each read done and reliable, and must agree before a barrier.
 // Returns true in that workgroup.
 __device__ __forceinline__ bool fold_finalise(const HopEpi& epi, const double* partial, int64_t nchunks, double* vl)
 {
@@ -317,7 +323,7 @@ __device__ __forceinline__ bool fold_finalise(const HopEpi& epi, const double* p
   CgState* fs = epi.st;
   if (!(fs->done || (epi.fold_pred == 1 && !fs->reliable) || (epi.fold_pred == 2 && fs->reliable))) {
     const double tot = block_sum_partials_256(partial, nchunks, vl);
-    if (threadIdx.x == 0) finalize(fs, epi.fold_fin, tot);
+    if (threadIdx.x == 0) finalize<true>(fs, epi.fold_fin, tot);
   }
   return true;
 }
@@ -340,7 +346,7 @@ __global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop(Geo g, i
   }
   const Map m = map_thread(S, g.Vh);
   CgState* st = epi.st ? epi.st + m.r : nullptr;
-  const bool skip = st && rhs_idle(st, epi.pred_reliable);
+  const bool skip = st && rhs_idle<MODE>(st, epi.pred_reliable);
   // a launch whose every right-hand side is idle does nothing (uniform over the grid)
   if (epi.st && S.NR == 1 && skip) return;
   double nrm = 0;
@@ -382,7 +388,7 @@ __global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop_lds(Geo 
   }
   const Map m = map_thread(S, g.Vh);
   CgState* st = epi.st ? epi.st + m.r : nullptr;
-  const bool skip = st && rhs_idle(st, epi.pred_reliable);
+  const bool skip = st && rhs_idle<MODE>(st, epi.pred_reliable);
   if (epi.st && skip) return;  // uniform: one right-hand side per launch
   const uint32_t e0 = (uint32_t)((m.chunk - (threadIdx.x >> 6)) * 64);  // first site of the workgroup
   const int t = (int)threadIdx.x;
@@ -428,7 +434,7 @@ __global__ void __launch_bounds__(256, 1) k_tm_hop_lds_p(Geo g, int op, SpinorVi
   using R = RealOf<SP>;
   __shared__ __attribute__((aligned(16))) char lds[Stage<SP, 12>::BYTES];
   CgState* st = epi.st;
-  if (st && rhs_idle(st, epi.pred_reliable)) return;  // uniform: one right-hand side per launch
+  if (st && rhs_idle<MODE>(st, epi.pred_reliable)) return;  // uniform: one right-hand side per launch
   const uint32_t b = blockIdx.x, nb = gridDim.x;
   const uint32_t xcd = b & 7u, bi = b >> 3;
   const int64_t nbx = (int64_t)(nb >> 3) + (xcd < (nb & 7u) ? 1 : 0);  // workgroups on this XCD
@@ -570,7 +576,7 @@ __global__ void __launch_bounds__(256, 2) k_tm_hop_split(Geo g, int op, SpinorVi
     if (fold_finalise(epi, partial, nchunks, (double*)xch)) return;
   }
   const CgState* st = epi.st;
-  if (st && rhs_idle(st, epi.pred_reliable)) return;  // uniform: one right-hand side per launch
+  if (st && rhs_idle<MODE>(st, epi.pred_reliable)) return;  // uniform: one right-hand side per launch
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t chunk = xcd_block();
   const bool active = chunk * 64 + lane < g.Vh;
@@ -687,7 +693,7 @@ __global__ void __launch_bounds__(256, 2) k_tm_hop_split_any(Geo g, int op, Spin
     if (fold_finalise(epi, partial, nchunks, (double*)xch)) return;
   }
   CgState* st = epi.st;
-  if (st && rhs_idle(st, epi.pred_reliable)) return;  // uniform: one right-hand side per launch
+  if (st && rhs_idle<MODE>(st, epi.pred_reliable)) return;  // uniform: one right-hand side per launch
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t chunk = xcd_block();
   const bool active = chunk * 64 + lane < g.Vh;
@@ -760,7 +766,7 @@ __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out
   unsigned busy = 0;
 #pragma unroll
   for (int b = 0; b < RB; b++)
-    if (b < nrb && !(epi.st && rhs_idle(epi.st + r0 + b, epi.pred_reliable))) busy |= 1u << b;
+    if (b < nrb && !(epi.st && rhs_idle<MODE>(epi.st + r0 + b, epi.pred_reliable))) busy |= 1u << b;
   // right-hand sides that idle here are skipped by the finalisation as well.
   // The busy right-hand sides' records of the workgroup's 256 sites are staged in LDS and
   // the neighbours among those sites read from there, as far as the LDS holds two
@@ -872,7 +878,7 @@ __global__ void __launch_bounds__(256, 2) k_tm_hop_rl(Geo g, int op, SpinorView 
   const int r0 = m.r * rpw, r1 = min(r0 + rpw, nr);
   unsigned busy = 0;
   for (int r = r0; r < r1; r++) {
-    if (epi.st && rhs_idle(epi.st + r, epi.pred_reliable)) {
+    if (epi.st && rhs_idle<MODE>(epi.st + r, epi.pred_reliable)) {
       if constexpr (MODE != 0) store_partial(0.0, partial, nchunks, r, m.chunk);
     } else {
       busy |= 1u << r;
