@@ -844,7 +844,7 @@ __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out
 // keeping the loop's loads unconditional matters: a load behind a branch makes every
 // later wait drain the queue (616 -> 546 us).
 // Slot K = 2 mu + (backward) of one FP16 neighbour applied to the accumulators.
-template <int K>
+template <int K, bool ANIS>
 __device__ __forceinline__ void rl_slot(const RawF16& w, const cx<float> u6[6], const float2* row2, float anis,
                                         cx<float> o[12])
 {
@@ -859,9 +859,14 @@ __device__ __forceinline__ void rl_slot(const RawF16& w, const cx<float> u6[6], 
   constexpr int MU = K / 2;
   constexpr bool FWD = (K & 1) == 0;
   cx<float> h0[3], h1[3], g0[3], g1[3];
-  project_f16<MU, FWD>(w, MU > 0 ? w.norm * anis : w.norm, h0, h1);
+  project_f16<MU, FWD>(w, w.norm, h0, h1);
   mat_vec(u, h0, g0);
   mat_vec(u, h1, g1);
+  // on the products, as hop_slot_rb has it: folded into the norm it rounds differently
+  if constexpr (MU > 0 && ANIS) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) { g0[c] = scal(g0[c], anis); g1[c] = scal(g1[c], anis); }
+  }
   scatter<float, MU, FWD>(o, g0, g1);
   // materialise the accumulators and keep the next loads behind this slot
 #pragma unroll
@@ -869,10 +874,12 @@ __device__ __forceinline__ void rl_slot(const RawF16& w, const cx<float> u6[6], 
   asm volatile("" ::: "memory");
 }
 
-template <int LK, int MODE, int XP, int CP>
+// ANIS: with an anisotropy factor (a branch on it in the loop costs every slot: twelve
+// right-hand sides at 16^3x32, solve 21.2 -> 21.4 ms)
+template <int LK, int MODE, int XP, int CP, bool ANIS>
 __global__ void __launch_bounds__(256, 2) k_tm_hop_rl(Geo g, int op, SpinorView out, SpinorView in, LinkView U,
-                                                      double anis_d, int use_anis, HopEpi epi, Shape S, int nr,
-                                                      int rpw, int64_t nchunks, double* partial)
+                                                      double anis_d, HopEpi epi, Shape S, int nr, int rpw,
+                                                      int64_t nchunks, double* partial)
 {
   const Map m = map_thread(S, g.Vh);
   const int r0 = m.r * rpw, r1 = min(r0 + rpw, nr);
@@ -898,7 +905,7 @@ __global__ void __launch_bounds__(256, 2) k_tm_hop_rl(Geo g, int op, SpinorView 
   cx<float> u[8][6];
 #pragma unroll
   for (int k = 0; k < 8; k++) Lk::load_stored(U.data[op], g.stride, k, e, u[k]);
-  const float anis = use_anis ? (float)anis_d : 1.f;
+  const float anis = (float)anis_d;
   constexpr int D = 4;  // neighbours in flight
   RawF16 w[D];
   int r = __builtin_ctz(busy);
@@ -922,7 +929,7 @@ __global__ void __launch_bounds__(256, 2) k_tm_hop_rl(Geo g, int op, SpinorView 
 #pragma unroll
     for (int k = 0; k < 12; k++) o[k] = mk<float>(0, 0);
 #define NQ_RL_SLOT(K)                                                              \
-  rl_slot<K>(w[K % D], u[K], row2, anis, o);                       \
+  rl_slot<K, ANIS>(w[K % D], u[K], row2, anis, o);                 \
   if (K + D < 8) w[K % D].load(in, g.stride, n[(K + D) % 8], r);                   \
   else w[K % D].load(in, g.stride, n[(K + D) % 8], rn);
     NQ_RL_SLOT(0) NQ_RL_SLOT(1) NQ_RL_SLOT(2) NQ_RL_SLOT(3)
@@ -1029,13 +1036,18 @@ static int launch_rl(nq_ctx* ctx, int op, const SpinorView& out, const SpinorVie
     sh.NRB = 1;
     sh.NRG = sh.NR = (nr + rpw - 1) / rpw;
     const dim3 grid((unsigned)(nblk * sh.NRG)), blk(256);
-    const int ua = anis != 1.0 ? 1 : 0;
-    if (links_stay(g, SP, LK, epi))
-      NQ_HOP_LAUNCH((k_tm_hop_rl<LK, MODE, XP, 0>), grid, blk, g, op, out, in, U, anis, ua, epi, sh, nr, rpw, nchunks,
-                    ctx->partial);
-    else
-      NQ_HOP_LAUNCH((k_tm_hop_rl<LK, MODE, XP, kNT>), grid, blk, g, op, out, in, U, anis, ua, epi, sh, nr, rpw,
-                    nchunks, ctx->partial);
+    const bool keep = links_stay(g, SP, LK, epi);
+#define NQ_RL(CP, ANIS)                                                                                             \
+  NQ_HOP_LAUNCH((k_tm_hop_rl<LK, MODE, XP, CP, ANIS>), grid, blk, g, op, out, in, U, anis, epi, sh, nr, rpw, nchunks, \
+                ctx->partial)
+    if (anis != 1.0) {
+      if (keep) NQ_RL(0, true);
+      else NQ_RL(kNT, true);
+    } else {
+      if (keep) NQ_RL(0, false);
+      else NQ_RL(kNT, false);
+    }
+#undef NQ_RL
     NQ_HIP(hipGetLastError());
     return NQ_OK;
   } else {

@@ -64,6 +64,28 @@ def test_batched_f16_kernels_agree(L, nr, prec, monkeypatch):
         assert np.array_equal(sols[0][i], sols[1][i]), i
 
 
+# an anisotropy factor scales the products of the x, y and z links: same bits from both
+# kernels, and alone as in the batch
+@pytest.mark.parametrize("L,nr", [((10, 4, 2, 2), 3), ((32, 16, 16, 16), 5)])
+@pytest.mark.parametrize("prec", ["f16", "f16h"])
+def test_batched_f16_kernels_agree_anisotropic(L, nr, prec, monkeypatch):
+    conf = conf_of(L, 57, [1.0, 0.2, 0, 0])
+    mus = [0.05 + 0.01 * i for i in range(nr)]
+    sols = []
+    for tune, n in (("0", nr), ("r", nr), ("r", 1)):
+        monkeypatch.setenv("NQ_TUNE", tune)
+        with nq.Ctx(L) as ctx:
+            g = nq.Gauge(ctx, lx=conf)
+            src = [ctx.field(nq.SPINCOLOR, nq.LX, nq.source_lx(L, 95 + i)) for i in range(n)]
+            sol = [ctx.field(nq.SPINCOLOR, nq.LX) for _ in range(n)]
+            res = nq.tm_solve_eoprec_multi(ctx, g, 0.16, mus[:n], 1000, 1e-14, sol, src, prec=prec, anis=0.87)
+            assert all(r["rc"] == nq.NQ_OK for r in res), res
+            sols.append([f.download() for f in sol])
+    for i in range(nr):
+        assert np.array_equal(sols[0][i], sols[1][i]), i
+    assert np.array_equal(sols[0][0], sols[2][0])
+
+
 @pytest.mark.parametrize("L", [(10, 4, 2, 2), (4, 6, 4, 10), (8, 4, 4, 12)])
 @pytest.mark.parametrize("theta", [[1.0, 0, 0, 0], [1.0, 0.3, -0.2, 0.5]])
 def test_f16_solves_with_phases(L, theta):
