@@ -189,4 +189,27 @@ NQ_HD inline void finalize(CgState* st, int fin, double total)
   record<RIDING>(st, fin, total);
 }
 
+// iterations to enqueue before the next poll, from the observed convergence rate: 2 to 64,
+// or last_chunk before there is one
+inline int next_chunk(double rr0, double rr, double target, int done_iters, int last_chunk)
+{
+  if (done_iters <= 0 || !(rr > 0) || !(rr0 > rr)) return last_chunk;
+  const double rate = std::log(rr / rr0) / done_iters;  // log decrease per iteration (<0)
+  const double need = std::ceil(std::log(target / rr) / rate) + 1;
+  return need < 2 ? 2 : (need < 64 ? (int)need : 64);  // 64 for a target of zero
+}
+
+// the same for a multi-shift solve with relative residuals: the running shift that needs
+// most (the targets are each shift's own, so that is not always the smallest shift)
+inline int next_chunk_cgm(const CgmState& s, int last_chunk)
+{
+  int n = 0;
+  for (int k = 0; k < s.nshift; k++) {
+    if (!s.run[k]) continue;
+    const int c = next_chunk(1.0, s.res[k], s.target[k], s.iter, last_chunk);
+    n = c > n ? c : n;
+  }
+  return n > 0 ? n : last_chunk;
+}
+
 }  // namespace nq

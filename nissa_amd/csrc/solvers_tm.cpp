@@ -171,18 +171,6 @@ static int get_states(nq_ctx* ctx, int i0, int n)
   return NQ_OK;
 }
 
-// iterations to enqueue before the next poll, from the observed convergence rate
-static int next_chunk(double rr0, double rr, double target, int done_iters, int last_chunk)
-{
-  if (done_iters <= 0 || !(rr > 0) || !(rr0 > rr)) return last_chunk;
-  const double rate = std::log(rr / rr0) / done_iters;  // log decrease per iteration (<0)
-  const double need = std::log(target / rr) / rate;
-  int n = (int)std::ceil(need) + 1;
-  if (n < 2) n = 2;
-  if (n > 64) n = 64;
-  return n;
-}
-
 struct Timer {
   hipEvent_t a = nullptr, b = nullptr;
   hipStream_t s;
@@ -1381,9 +1369,7 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
   // alpha (-betaa) and the stop flag of the source, for the hop epilogues
   NQ_TRY(put_state(ctx, 0, CgState{}));
   CgState* mirror = ctx->state;
-  int chunk = 8, launched = 0, kref = 0;
-  for (int k = 1; k < nmass; k++)
-    if (masses[k] * masses[k] < masses[kref] * masses[kref]) kref = k;
+  int chunk = 8, launched = 0;
   for (;;) {
     for (int it = 0; it < chunk; it++) {
       NQ_TRY(q2_first(ctx, Q, 0.0, &ft, &fp, mirror));  // t = Q(0) p, |t|^2
@@ -1397,8 +1383,7 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
     NQ_HIP(hipStreamSynchronize(ctx->stream));
     if (hst->nan) return fail(NQ_ENAN, "nanned");
     if (hst->done || launched > niter + 64) break;
-    // the shift of the smallest mass converges last
-    chunk = next_chunk(1.0, hst->res[kref], residues[kref], hst->iter, std::min(64, chunk * 2));
+    chunk = next_chunk_cgm(*hst, std::min(64, chunk * 2));
   }
   const int iters = hst->iter;
   // copy out and the FP64 check |(Q(-m)Q(+m)) x_k - b|^2 / |b|^2

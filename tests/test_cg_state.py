@@ -3,6 +3,8 @@
 A finalisation that rides in a hop shares its launch with workgroups that read `done` and
 `reliable`.  It must leave both words alone, raise the same bits in `stop`, and agree with
 the finalisation launched by itself in every other field.
+
+The poll interval of a multi-shift solve follows the running shift that needs most.
 """
 import os
 import shutil
@@ -44,6 +46,34 @@ int main()
 """
 
 
+# smallest mass first; it has the looser residue and has stopped
+POLL = r"""
+#include <cstdio>
+#include <cstring>
+#include "cg_state.hpp"
+using namespace nq;
+
+int main()
+{
+  CgmState s;
+  std::memset(&s, 0, sizeof s);
+  s.nshift = 2; s.iter = 40;
+  s.run[1] = 1;
+  s.res[0] = 9e-5; s.target[0] = 1e-4;
+  s.res[1] = 1e-10; s.target[1] = 1e-12;
+  std::printf("%d\n", next_chunk_cgm(s, 16));  // 40 iterations for ten decades: 8 for two, and one
+  s.target[1] = 0;
+  std::printf("%d\n", next_chunk_cgm(s, 16));
+  s.run[0] = 1; s.res[0] = 1e-3; s.target[1] = 1e-12;  // both run: 14 for the first
+  std::printf("%d\n", next_chunk_cgm(s, 16));
+  s.res[0] = 2;  // no estimate for it yet
+  std::printf("%d\n", next_chunk_cgm(s, 16));
+  s.run[0] = s.run[1] = 0;
+  std::printf("%d\n", next_chunk_cgm(s, 16));
+}
+"""
+
+
 def run_host(tmp_path, source):
     (tmp_path / "t.cpp").write_text(source)
     exe = str(tmp_path / "t")
@@ -58,3 +88,8 @@ def test_riding_finalisation_leaves_done_and_reliable(tmp_path):
     assert len(out) == 21 and all(l[0] == "1" and l[1] == "1" for l in out), out
     # nothing pending: only <p, A p> can stop; a plain and a mixed CG with |r|^2 pending
     assert [int(l[2]) for l in out] == [0, 0, 0, 0, 0, 1, 1] + [0, 1, 0, 1, 1, 1, 1] + [0, 2, 2, 2, 1, 1, 1], out
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host C++ compiler")
+def test_poll_interval_of_a_multi_shift_solve(tmp_path):
+    assert [int(l[0]) for l in run_host(tmp_path, POLL)] == [9, 64, 15, 16, 16]
