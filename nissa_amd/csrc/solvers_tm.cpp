@@ -1300,8 +1300,7 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
                       double* true_res)
 {
   const int64_t fsz = 24 * ctx->geo.stride;  // elements of one lx field
-  SpinorView rv, pv, tv, sv, qv, ps, xs;
-  NQ_TRY(alloc_spinor_nr(ctx, "q2m.rprev", SP_F64, 24, 1, &qv));
+  SpinorView rv, pv, tv, sv, ps, xs;
   NQ_TRY(alloc_spinor_nr(ctx, "q2.r", SP_F64, 12, 2, &rv));
   NQ_TRY(alloc_spinor_nr(ctx, "q2.p", SP_F64, 12, 2, &pv));
   NQ_TRY(alloc_spinor_nr(ctx, "q2.t", SP_F64, 12, 2, &tv));
@@ -1325,6 +1324,8 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
     }
   } rel{{&fr, &fp, &ft, &fs}};
   const SpinorView b = view_lx_flat(src), r = view_lx_flat(&fr), p = view_lx_flat(&fp), s = view_lx_flat(&fs);
+  // s is needed for the final check only: until then it keeps the pending iteration's r
+  const SpinorView& rprev = s;
   SpinorView none;
   none.ncomp = 24;
   Timer T(ctx->stream);
@@ -1376,7 +1377,7 @@ static int q2_cgm_f64(nq_ctx* ctx, const ApplyQ& Q, int nmass, const double* mas
       NQ_TRY(launch_cgm_finalize_lx(ctx, dst, 1, mirror));  // pap = |t|^2
       NQ_TRY(q2_second(ctx, Q, 0.0, &ft, &fr, &fp, nullptr, mirror));  // r += betaa Q(0) t, |r|^2
       NQ_TRY(launch_cgm_finalize_lx(ctx, dst, 2, mirror));
-      NQ_TRY(launch_cgm_vec(ctx, r, qv, p, xs, ps, fsz, dst, nmass));
+      NQ_TRY(launch_cgm_vec(ctx, r, rprev, p, xs, ps, fsz, dst, nmass));
     }
     launched += chunk;
     NQ_HIP(hipMemcpyAsync(hst, dst, sizeof(CgmState), hipMemcpyDeviceToHost, ctx->stream));
