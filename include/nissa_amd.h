@@ -68,7 +68,8 @@ int nq_device_count(int* n);
    timing the hops on synthetic data at creation, or read from the tile cache that run
    wrote (NQ_TUNE_CACHE, else $HOME/.cache/nissa_amd/site_tiles.txt), as nissa's kernel
    tuner keeps its table on disk (src/threads/benchmarks.hpp:118-200,207-328).
-   NQ_TTILE / NQ_XYTILE fix the tiles, NQ_TUNE_TILES=0 keeps the defaults.  The order
+   NQ_TTILE / NQ_XYTILE fix the tiles, NQ_TUNE_TILES=0 keeps the defaults; NQ_ZTILE sets
+   the z tile, for which the others are chosen.  The order
    changes global sums at the rounding level only. */
 int nq_ctx_create(int T, int LX, int LY, int LZ, int device, nq_ctx** out);
 void nq_ctx_destroy(nq_ctx* ctx);

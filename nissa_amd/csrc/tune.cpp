@@ -8,10 +8,11 @@
 // constant synthetic conf for each candidate order, times the FP64 hop and the FP16
 // hop (the plain solve's and the mixed solve's dominant kernels; their run time does
 // not depend on the values), and keeps the order with the smallest sum.  The choice is
-// appended to a cache file, one line per device architecture and lattice
-//   <arch> <T> <LX> <LY> <LZ> <TB> <TX> <TY> <us FP64 hop> <us FP16 hop>
+// appended to a cache file, one line per device architecture, lattice and z tile
+//   <arch> <T> <LX> <LY> <LZ> <TB> <TX> <TY> <us FP64 hop> <us FP16 hop> <TZ>
 // (NQ_TUNE_CACHE, else $HOME/.cache/nissa_amd/site_tiles.txt; the last matching
 // line wins), so later contexts of that lattice read it instead of timing again.
+// Lines without a z tile were timed on an order that had none and are passed over.
 // Lattices under 2^18 sites per parity keep the default order, and NQ_TUNE_TILES=0
 // switches the tuner off.  Every candidate computes each site exactly as the default
 // order does; only the order of the global sums changes, so a result depends on the
@@ -46,7 +47,7 @@ std::map<std::string, std::array<int, 3>> g_seen;
 std::string key_of(const std::string& arch, const Geo& g)
 {
   return arch + " " + std::to_string(g.T) + " " + std::to_string(g.LX) + " " + std::to_string(g.LY) + " " +
-         std::to_string(g.LZ);
+         std::to_string(g.LZ) + " " + std::to_string(g.TZ);
 }
 
 std::string cache_path()
@@ -77,9 +78,9 @@ bool cache_lookup(const std::string& path, const std::string& arch, const Geo& g
   char line[256], a[64];
   bool found = false;
   while (fgets(line, sizeof line, f)) {
-    int T, X, Y, Z, b, x, y;
-    if (sscanf(line, "%63s %d %d %d %d %d %d %d", a, &T, &X, &Y, &Z, &b, &x, &y) != 8) continue;
-    if (arch == a && T == g.T && X == g.LX && Y == g.LY && Z == g.LZ && b >= 2 && g.T % b == 0 && x >= 1 &&
+    int T, X, Y, Z, b, x, y, z;
+    if (sscanf(line, "%63s %d %d %d %d %d %d %d %*f %*f %d", a, &T, &X, &Y, &Z, &b, &x, &y, &z) != 9) continue;
+    if (arch == a && T == g.T && X == g.LX && Y == g.LY && Z == g.LZ && z == g.TZ && b >= 2 && g.T % b == 0 && x >= 1 &&
         g.LX % x == 0 && y >= 1 && g.LY % y == 0) {
       *tb = b;
       *tx = x;
@@ -97,8 +98,8 @@ void cache_store(const std::string& path, const std::string& arch, const Geo& g,
   FILE* f = fopen(path.c_str(), "a");
   if (!f) return;
   char line[256];
-  const int n = snprintf(line, sizeof line, "%s %d %d %d %d %d %d %d %.1f %.1f\n", arch.c_str(), g.T, g.LX, g.LY,
-                         g.LZ, g.TB, g.TX, g.TY, us64, us16);
+  const int n = snprintf(line, sizeof line, "%s %d %d %d %d %d %d %d %.1f %.1f %d\n", arch.c_str(), g.T, g.LX,
+                         g.LY, g.LZ, g.TB, g.TX, g.TY, us64, us16, g.TZ);
   if (n > 0) fwrite(line, 1, (size_t)n, f);  // one write per line: appends of several processes stay whole
   fclose(f);
 }
