@@ -12,6 +12,7 @@
 
 #include "../../include/nissa_amd.h"
 #include "cg_state.hpp"
+#include "hop_rules.hpp"
 
 namespace nq {
 
@@ -28,13 +29,6 @@ int fail(int code, const char* fmt, ...);
     int rc_ = (call);           \
     if (rc_ != NQ_OK) return rc_; \
   } while (0)
-
-// ---------------------------------------------------------------- storage kinds
-enum SpPrec { SP_F64 = 0, SP_F32 = 1, SP_F16 = 2 };
-enum LkPrec { LK_F64_18 = 0, LK_F32_18 = 1, LK_F32_12 = 2, LK_F16_12 = 3, LK_F64_12 = 4 };
-// complex elements stored per link (12-real: rows 0 and 1) and bytes per element
-constexpr int lk_nc(int lk) { return (lk == LK_F64_18 || lk == LK_F32_18) ? 9 : 6; }
-constexpr int lk_eb(int lk) { return (lk == LK_F64_18 || lk == LK_F64_12) ? 16 : (lk == LK_F16_12 ? 4 : 8); }
 
 // Device geometry of one lattice (all extents even).
 // Device site order: (th, xt, yt, zt, xi, yi, zi, tl) from slowest to fastest, with

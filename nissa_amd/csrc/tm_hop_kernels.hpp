@@ -975,50 +975,6 @@ static int launch_rb(nq_ctx* ctx, int RB, int op, const SpinorView& out, const S
   return NQ_OK;
 }
 
-// Whether the links and the data used once are accessed with the default cache policy,
-// to be found in the 256 MB memory-side cache by the next hop, instead of streamed past
-// it: when the links of both parities (and the clover blocks of K) and the input and
-// output spinors take at most 224 MB (150 MB for several right-hand sides, whose other
-// vectors grow with them).  Measured, default against streamed, whole solves
-// (links of both parities): 123 MB (FP16 inner, 20^3x40) 7.41 against 8.23 ms, 127 MB
-// (FP16 links, 24^3x48) 11.6 / 12.7, 151 MB (FP64, 16^3x32) 7.56 / 8.03, 184 MB (FP32,
-// 20^3x40) 9.35 / 10.2; above it 236 MB (FP16 links, 28^3x56) 22.0 / 21.2, 255 MB (FP16
-// inner, 24^3x48) 14.5 / 14.1, 369 MB (FP64, 20^3x40) 19.9 / 19.0, 805 MB (FP16 inner,
-// 32^3x64) 41.2 / 37.4.  Twelve FP16 right-hand sides: 50 MB of links 21.8 / 22.1, 123 MB
-// (and 200 MB of spinors) 56.6 / 54.6, 255 MB 114.6 / 108.6; five at 46x16x22x20, 124 and
-// 84 MB, 26.4 / 25.9.
-inline bool links_stay(const Geo& g, int sp, int lk, const HopEpi& epi)
-{
-  const int eb = sp == SP_F64 ? 16 : (sp == SP_F32 ? 8 : 4);
-  double site = 2.0 * 8 * lk_nc(lk) * lk_eb(lk) + 2.0 * 12 * eb * epi.nrhs;
-  if (epi.blk_mode) site += (72 + 36) * eb;
-  return site * (double)g.Vh <= (epi.nrhs > 1 ? 150.0 : 224.0) * 1048576;
-}
-
-// Neighbours staged in LDS (k_tm_hop_lds) for one right-hand side: FP64 always (4 % at
-// 32^3x64), the sloppy precisions when the links are streamed: unstaged against staged,
-// FP32 54.4 / 49.8 us at 24^3x48 and 139 / 132 at 32^3x64; FP16 34.1 / 33.4 and 91 / 86;
-// FP16 links at 32^3x64 66.5 / 63.5.  With the links in the memory-side cache the staging
-// round trip is not paid back: 16^3x32 FP32 10.7 / 12.0 us, FP16 9.4 / 10.1, FP16 links
-// 9.1 / 9.7; 24^3x48, FP16 links 24.1 / 25.6.
-inline bool use_lds(int sp, bool keep) { return sp == SP_F64 || !keep; }
-
-// Hops of one right-hand side split the directions over the wavefronts of a workgroup
-// (k_tm_hop_split and k_tm_hop_split_any) on lattices below a number of sites per parity.
-// Plain FP64 below 2^18, where the persistent kernel does not fill its slots twice; one
-// thread per site / split: hop on 8^4 10.3 / 4.6 us, 12x6x10x14 14.5 / 4.7, 24x12^3 16.6 /
-// 7.4, 16^3x32 20.2 / 18.6, 20^3x40 55.0 / 48.6; above, 24^3x48 98 / 103, 28^3x56 177 / 190.
-// The others finish a site in one wavefront of four and lose sooner.  Sloppy precisions
-// below 2^17: FP16 inner solves at 8^3x16 3.22 / 2.35 ms, 24x12^3 3.52 / 2.65, 16^3x32 4.42 /
-// 3.95 (FP32 4.49 / 4.31), 20^3x40 6.95 / 6.98.  Clover blocks, FP16 and FP32 below 2^15:
-// 24x12^3 3.89 / 3.06 ms, 16^3x32 4.92 / 5.21; FP64 below 2^13: 8^3x16 3.76 / 3.18 ms,
-// 24x12^3 4.67 / 5.20.
-inline bool use_split(const Geo& g, int sp, bool plain64, bool clover)
-{
-  const int bits = plain64 ? 18 : (!clover ? 17 : (sp == SP_F64 ? 13 : 15));
-  return g.Vh < (int64_t(1) << bits);
-}
-
 // launch of k_tm_hop_rl: the right-hand sides split into the fewest groups that give
 // every CU its two resident workgroups (16^3x32, 12 right-hand sides: one group 42.5 us,
 // two 34.5, three 36.5; 24^3x48: one group 193 us, two 198, three 205).
@@ -1036,7 +992,7 @@ static int launch_rl(nq_ctx* ctx, int op, const SpinorView& out, const SpinorVie
     sh.NRB = 1;
     sh.NRG = sh.NR = (nr + rpw - 1) / rpw;
     const dim3 grid((unsigned)(nblk * sh.NRG)), blk(256);
-    const bool keep = links_stay(g, SP, LK, epi);
+    const bool keep = links_stay(g.Vh, SP, LK, nr, false);
 #define NQ_RL(CP, ANIS)                                                                                             \
   NQ_HOP_LAUNCH((k_tm_hop_rl<LK, MODE, XP, CP, ANIS>), grid, blk, g, op, out, in, U, anis, epi, sh, nr, rpw, nchunks, \
                 ctx->partial)
@@ -1196,11 +1152,11 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
   if (!fold_here) ke.fold_fin = FIN_NONE;
   const dim3 grid((unsigned)(L.blocks + (fold_here ? 1 : 0))), blk(L.threads);
   const int ua = anis != 1.0 ? 1 : 0;
-  const bool keep = links_stay(g, SP, LK, epi);
-  const bool lds_ok = nr == 1 && L.s.W == 4 && !(lenv && lenv[0] == '0') && use_lds(SP, keep);
-  // the specialised FP64 kernel has no precision conversion and no clover blocks
-  constexpr bool plain64 = SP == SP_F64 && XP == SP_F64 && CLV == 0;
-  if (nr == 1 && !epi.coef && use_split(g, SP, plain64, CLV != 0)) {
+  const HopRoute route = hop_route(g.Vh, SP, LK, XP, CLV != 0, nr, epi.coef != nullptr, !(lenv && lenv[0] == '0'));
+  const bool keep = route.keep, lds_ok = route.kernel == HOP_LDS;
+  if (route.kernel == HOP_SPLIT) {
+    // the specialised FP64 kernel has no precision conversion and no clover blocks
+    constexpr bool plain64 = SP == SP_F64 && XP == SP_F64 && CLV == 0;
     HopEpi ks = epi;
     fold_here = MODE == 0 && epi.fold_fin != FIN_NONE && epi.st;
     if (!fold_here) ks.fold_fin = FIN_NONE;
@@ -1212,8 +1168,14 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
       else
         NQ_HOP_LAUNCH((k_tm_hop_split<LK, MODE, kNT>), sg, dim3(256), g, op, out, in, U, anis, ua, ks, L.nchunks, part);
     } else {
-      NQ_HOP_LAUNCH((k_tm_hop_split_any<SP, LK, MODE, XP, CLV, 0>), sg, dim3(256), g, op, out, in, U, anis, ua, ks,
-                    L.nchunks, part);
+      // links that do not stay: only those of the FP64 residual hop, on the lattices split here
+      constexpr int NK = SP == SP_F64 && MODE == 3 ? kNT : 0;
+      if (keep)
+        NQ_HOP_LAUNCH((k_tm_hop_split_any<SP, LK, MODE, XP, CLV, 0>), sg, dim3(256), g, op, out, in, U, anis, ua, ks,
+                      L.nchunks, part);
+      else
+        NQ_HOP_LAUNCH((k_tm_hop_split_any<SP, LK, MODE, XP, CLV, NK>), sg, dim3(256), g, op, out, in, U, anis, ua, ks,
+                      L.nchunks, part);
     }
     prof_end_ext(ctx);
     NQ_HIP(hipGetLastError());

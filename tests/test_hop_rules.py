@@ -1,0 +1,60 @@
+"""Kernel and cache policy of the twisted-mass hop (csrc/hop_rules.hpp), built by a host
+compiler and walked over lattices, precisions and link kinds."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nissa_amd", "csrc")
+
+SRC = r"""
+#include <cstdio>
+#include "hop_rules.hpp"
+using namespace nq;
+
+int main()
+{
+  // spinor, link and tail precisions of the instances; clover blocks; batched residual
+  const struct { int sp, lk, xp, clover, per_rhs; } inst[] = {
+      {SP_F64, LK_F64_18, SP_F64, 0, 0}, {SP_F64, LK_F64_12, SP_F64, 0, 0}, {SP_F64, LK_F64_18, SP_F32, 0, 0},
+      {SP_F64, LK_F64_12, SP_F32, 0, 0}, {SP_F64, LK_F64_18, SP_F64, 1, 0}, {SP_F32, LK_F32_18, SP_F32, 0, 0},
+      {SP_F32, LK_F32_18, SP_F32, 1, 0}, {SP_F16, LK_F32_12, SP_F32, 0, 0}, {SP_F16, LK_F32_12, SP_F32, 1, 0},
+      {SP_F16, LK_F16_12, SP_F32, 0, 0}, {SP_F16, LK_F16_12, SP_F32, 1, 0}, {SP_F64, LK_F64_18, SP_F32, 0, 1},
+      {SP_F64, LK_F64_12, SP_F32, 0, 1}};
+  for (auto& i : inst)
+    for (int64_t Vh = 8; Vh < (int64_t(1) << 22); Vh += 1 + Vh / 200) {
+      const HopRoute r = hop_route(Vh, i.sp, i.lk, i.xp, i.clover, 1, i.per_rhs, true);
+      std::printf("%d %d %d %d %d %lld %d %d\n", i.sp, i.lk, i.xp, i.clover, i.per_rhs, (long long)Vh, r.kernel, r.keep);
+    }
+}
+"""
+F64, F32, F16 = 0, 1, 2
+LINK = {0: 144, 1: 72, 2: 48, 3: 24, 4: 96}  # bytes of a link
+PLAIN, LDS, SPLIT = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def routes(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("no host C++ compiler")
+    d = tmp_path_factory.mktemp("rules")
+    (d / "t.cpp").write_text(SRC)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Wextra", "-Werror", "-I", CSRC, str(d / "t.cpp"), "-o", str(d / "t")],
+                   check=True)
+    out = subprocess.run([str(d / "t")], check=True, capture_output=True, text=True).stdout
+    return [tuple(int(v) for v in l.split()) for l in out.splitlines()]
+
+
+def test_one_policy_for_every_kernel(routes):
+    """Default cache policy when links, clover blocks, input and output fit 224 MB, whichever
+    kernel runs: split ones too, among which only the FP64 residual hop can exceed it."""
+    seen = set()
+    for sp, lk, xp, clover, per_rhs, Vh, kernel, keep in routes:
+        eb = {F64: 16, F32: 8, F16: 4}[sp]
+        site = 16 * LINK[lk] + 24 * eb + (108 * eb if clover else 0)
+        assert keep == (site * Vh <= 224 << 20), (sp, lk, Vh)
+        if kernel == SPLIT and not keep and (sp, xp, clover) != (F64, F64, 0):
+            assert (sp, xp, clover) == (F64, F32, 0)
+            seen.add(lk)
+    assert seen == {0, 4}
