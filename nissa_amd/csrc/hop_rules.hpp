@@ -79,4 +79,9 @@ inline HopRoute hop_route(int64_t Vh, int sp, int lk, int xp, bool clover, int n
   return r;
 }
 
+// Whether HOP_LDS can come with keep: the sloppy precisions stage streamed links only, and a
+// plain FP64 hop that is not split (2^18 sites) exceeds the 224 MB.  Not so the clover hops
+// and, in a batch, the residual (mode 3).
+constexpr bool hop_lds_keeps(int sp, int mode, bool clover) { return sp == SP_F64 && (mode == 3 || clover); }
+
 }  // namespace nq

@@ -1183,10 +1183,12 @@ static int go(nq_ctx* ctx, int op, const SpinorView& out, const SpinorView& in, 
     if (MODE != 0 && epi.fin != FIN_PARTIAL) NQ_TRY(launch_finalize(ctx, nr, epi.st, epi.fin, epi.pred_reliable));
     return NQ_OK;
   }
+  // with the default policy only where hop_route can come to it
+  constexpr int KL = hop_lds_keeps(SP, MODE, CLV != 0) ? 0 : kNT;
   if (lds_ok && launch_persistent<SP, LK, MODE, XP, CLV>(ctx, op, out, in, U, anis, epi, L)) {
     fold_here = false;
   } else if (lds_ok && keep) {
-    NQ_HOP_LAUNCH((k_tm_hop_lds<SP, LK, MODE, XP, CLV, 0>), grid, blk, g, op, out, in, U, anis, ua, ke, L.s, L.nchunks,
+    NQ_HOP_LAUNCH((k_tm_hop_lds<SP, LK, MODE, XP, CLV, KL>), grid, blk, g, op, out, in, U, anis, ua, ke, L.s, L.nchunks,
                   ctx->partial + epi.part0);
   } else if (lds_ok) {
     NQ_HOP_LAUNCH((k_tm_hop_lds<SP, LK, MODE, XP, CLV, kNT>), grid, blk, g, op, out, in, U, anis, ua, ke, L.s,

@@ -58,3 +58,10 @@ def test_one_policy_for_every_kernel(routes):
             assert (sp, xp, clover) == (F64, F32, 0)
             seen.add(lk)
     assert seen == {0, 4}
+
+
+def test_staged_hops_that_keep_their_links(routes):
+    """The instances left out (hop_lds_keeps) are those that no lattice comes to: staging with
+    the default policy happens in FP64 clover hops and batched residuals only."""
+    kept = {(sp, clover, per_rhs) for sp, lk, xp, clover, per_rhs, Vh, kernel, keep in routes if kernel == LDS and keep}
+    assert kept == {(F64, 1, 0), (F64, 0, 1)}
