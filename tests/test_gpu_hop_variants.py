@@ -170,3 +170,55 @@ def test_staggered_batch_same_bits_whatever_the_block(L, nr, prec, monkeypatch):
             out[rb] = np.stack([f.download() for s in sol for f in s])
     for rb in ("1", "4", "6"):
         assert np.array_equal(out[None], out[rb]), rb
+
+
+def test_persistent_hop_against_oracle(monkeypatch):
+    """32^4: 2048 blocks, at least twice the slots of 256 CUs that hold up to four workgroups
+    of 48 KB of LDS in 160 KB, and too large to be split: the persistent FP64 hop, both
+    parities against the oracle, and the one-shot kernel's bits."""
+    L = (32, 32, 32, 32)
+    conf = conf_of(L, 58, [1.0, 0, 0, 0])
+    geo = orc.Geom(L)
+    ce, co = geo.split(conf)
+    x = gauss_eo(geo.Vh, 12)
+    with nq.Ctx(L) as ctx:
+        g = nq.Gauge(ctx, lx=conf)
+        for out_par in (0, 1):
+            fi, fo = ctx.field(nq.SPINCOLOR, 1 - out_par, x), ctx.field(nq.SPINCOLOR, out_par)
+            monkeypatch.setenv("NQ_PERSIST", "1")
+            nq.tm_hop(ctx, g, fo, fi)
+            hop = fo.download()
+            assert rel_l2(hop, geo.tm_hop(out_par, ce, co, x)) < 1e-14
+            monkeypatch.setenv("NQ_PERSIST", "0")
+            nq.tm_hop(ctx, g, fo, fi)
+            assert np.array_equal(fo.download(), hop)
+
+
+# links past the memory-side cache: the one-source hops with clover blocks are staged in LDS
+# (NQ_LDS=0: they are not), and a batch runs the plain ones
+@pytest.mark.parametrize("prec", ["f16", "f16h", "f32"])
+def test_clover_with_streamed_links(prec, monkeypatch):
+    L, kappa, mu, n = (48, 24, 24, 24), 0.13, 0.05, 3
+    conf = conf_of(L, 59, [1.0, 0, 0, 0])
+    with nq.Ctx(L) as ctx:
+        g = nq.Gauge(ctx, lx=conf)
+        cl = nq.Clover(ctx, g, 1.0)
+        src = [ctx.field(nq.SPINCOLOR, nq.LX, nq.source_lx(L, 75 + i)) for i in range(n)]
+        sol = [ctx.field(nq.SPINCOLOR, nq.LX) for _ in src]
+        out = []
+        for lds in ("1", "0"):
+            monkeypatch.setenv("NQ_LDS", lds)
+            st = nq.tmclov_solve_eoprec(ctx, g, cl, kappa, mu, 1000, 1e-14, sol[0], src[0], prec=prec)
+            assert st["rc"] == nq.NQ_OK and st["rel_res_sq"] < 1e-14, st
+            out.append(sol[0].download())
+        assert np.array_equal(out[0], out[1])
+        monkeypatch.delenv("NQ_LDS")
+        res = nq.tmclov_solve_eoprec_multi(ctx, g, cl, kappa, mu, 1000, 1e-14, sol, src, prec=prec)
+        assert all(r["rc"] == nq.NQ_OK and r["rel_res_sq"] < 1e-14 for r in res), res
+        batch = [f.download() for f in sol]
+        # |x - y| <= |(K K^+)^-1| (|r_x| + |r_y|) with |r| = 1e-7 |b| each; the smallest
+        # eigenvalue of K K^+ is at least (2 kappa mu)^2 in units of the largest
+        assert rel_l2(batch[0], out[0]) < 2e-7 / (2 * kappa * mu) ** 2
+        one = [ctx.field(nq.SPINCOLOR, nq.LX)]
+        nq.tmclov_solve_eoprec_multi(ctx, g, cl, kappa, mu, 1000, 1e-14, one, src[2:], prec=prec)
+        assert np.array_equal(one[0].download(), batch[2])
