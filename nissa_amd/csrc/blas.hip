@@ -146,36 +146,40 @@ __device__ __forceinline__ bool rr_inline(const BlasArgs& A, double* vl, double*
   return !(isnan(tot) || sqrt(tot) < s->delta * s->r0 || tot < s->target || last);
 }
 
-// Whether the p update of right-hand side m.r idles.  A stop that a finalisation riding in a
-// hop left (CgState::stop) becomes done / reliable here: with it set, no workgroup of this
-// launch reads those two.
+// Whether the p update of right-hand side m.r idles.  Where (FIN) it takes the place of the
+// finalisation of |r|^2, a stop that a finalisation riding in a hop left (CgState::stop)
+// becomes done / reliable here: with it set, no workgroup of this launch reads those two.
+template <bool FIN>
 __device__ __forceinline__ bool pupdate_idle(const BlasArgs& A, const Map& m)
 {
   CgState* s = A.st + m.r;
-  const int stop = s->stop;
-  if (stop) {
-    if (m.chunk == 0 && (threadIdx.x & 63) == 0) raise_stop<false>(s, stop);
-    return true;
+  if constexpr (FIN) {
+    const int stop = s->stop;
+    if (stop) {
+      if (m.chunk == 0 && (threadIdx.x & 63) == 0) raise_stop<false>(s, stop);
+      return true;
+    }
   }
-  return s->done || (A.pred == 2 ? !s->reliable : s->reliable);
+  const int reliable = sload(&s->reliable);
+  return sload(&s->done) || (A.pred == 2 ? !reliable : reliable);
 }
 
 // p = r + beta p, beta from state[r]; skipped once that right-hand side is done or
 // while it waits for a reliable update.  With x given, first x += alpha p (the CG
 // solution update moved out of the matvec tail, so that p is read once per
 // iteration)
-template <int NC>
+template <int NC, bool FIN = false>
 __global__ void __launch_bounds__(256) k_pupdate(BlasArgs A, SpinorView p, SpinorView r, SpinorView x)
 {
   const Map m = map_thread(A.s, A.g.Vh);
   const CgState* s = A.st + m.r;
-  if (pupdate_idle(A, m)) return;  // uniform per right-hand side
+  if (pupdate_idle<FIN>(A, m)) return;  // uniform per right-hand side
   double beta;
-  if (A.fin != FIN_NONE) {
+  if constexpr (FIN) {
     __shared__ double vl[1024];
     if (!rr_inline(A, vl, &beta)) return;  // one right-hand side: uniform over the workgroup
   } else {
-    beta = s->beta;
+    beta = sload(&s->beta);
   }
   if (!m.active) return;
   cx<double> pv[NC], rv[NC];
@@ -205,22 +209,22 @@ __global__ void __launch_bounds__(256) k_pupdate(BlasArgs A, SpinorView p, Spino
 // x += alpha_prev p_prev + alpha p_in, p_prev being the previous iteration's p still in
 // p_out: x is read and written half as often, and the x terms of an iteration that
 // does not apply them wait in p_out until the next one.
-template <int NC>
+template <int NC, bool FIN = false>
 __global__ void __launch_bounds__(256) k_pupdate_pair(BlasArgs A, SpinorView pin, SpinorView pout, SpinorView r,
                                                       SpinorView x)
 {
   const Map m = map_thread(A.s, A.g.Vh);
   const CgState* s = A.st + m.r;
-  if (pupdate_idle(A, m)) return;
+  if (pupdate_idle<FIN>(A, m)) return;
   double beta;
   bool xstep;
-  if (A.fin != FIN_NONE) {
+  if constexpr (FIN) {
     __shared__ double vl[1024];
     if (!rr_inline(A, vl, &beta)) return;  // uniform over the workgroup
     xstep = s->xlag != 0;  // the xstep that recording this finalisation will set
   } else {
-    beta = s->beta;
-    xstep = s->xstep != 0;
+    beta = sload(&s->beta);
+    xstep = sload(&s->xstep) != 0;
   }
   if (!m.active) return;
   cx<double> pv[NC], rv[NC];
@@ -328,7 +332,12 @@ __global__ void __launch_bounds__(1024) k_finalize(const double* partial, int64_
   __shared__ double vl[1024];
   CgState* s = st + blockIdx.x;
   // uniform over the workgroup
-  if (s->stop || s->done || (pred_reliable == 1 && !s->reliable) || (pred_reliable == 2 && s->reliable)) return;
+  const int stop = s->stop;
+  if (stop) {  // left by a finalisation riding in a hop: done / reliable from here on
+    if (threadIdx.x == 0) raise_stop<false>(s, stop);
+    return;
+  }
+  if (s->done || (pred_reliable == 1 && !s->reliable) || (pred_reliable == 2 && s->reliable)) return;
   const double tot = block_sum_partials(partial + (int64_t)blockIdx.x * nchunks, nchunks, vl);
   if (threadIdx.x == 0) finalize(s, fin, tot);
 }
@@ -462,7 +471,8 @@ int launch_cg_pupdate(nq_ctx* ctx, const SpinorView& p, const SpinorView& r, CgS
   BlasArgs A;
   Launch L;
   NQ_TRY(make_args(ctx, nr, st, fin, pred == 2 ? 2 : 1, &A, &L));
-  if (fin != FIN_NONE && (nr != 1 || L.threads != 256 || pred != 1 || (fin != FIN_RR && fin != FIN_RR_SLOPPY)))
+  if (fin != FIN_NONE &&
+      (nr != 1 || L.threads != 256 || pred != 1 || p.ncomp != 12 || (fin != FIN_RR && fin != FIN_RR_SLOPPY)))
     return fail(NQ_EINVAL, "pupdate: finalisation %d needs one right-hand side", fin);
   if (x.data && x.ncomp != p.ncomp) return fail(NQ_EINVAL, "pupdate: component mismatch");
   hipEvent_t ev = nullptr;
@@ -470,7 +480,8 @@ int launch_cg_pupdate(nq_ctx* ctx, const SpinorView& p, const SpinorView& r, CgS
   prof_begin(ctx, x.data ? "blas_xpupdate" : "blas_pupdate",
              nr * (2 * site_bytes(p) + site_bytes(r) + xb) * (double)ctx->geo.Vh, &ev);
   const dim3 grid((unsigned)L.blocks), blk(L.threads);
-  if (p.ncomp == 24) hipLaunchKernelGGL(k_pupdate<24>, grid, blk, 0, ctx->stream, A, p, r, x);
+  if (fin != FIN_NONE) hipLaunchKernelGGL((k_pupdate<12, true>), grid, blk, 0, ctx->stream, A, p, r, x);
+  else if (p.ncomp == 24) hipLaunchKernelGGL(k_pupdate<24>, grid, blk, 0, ctx->stream, A, p, r, x);
   else if (p.ncomp == 12) hipLaunchKernelGGL(k_pupdate<12>, grid, blk, 0, ctx->stream, A, p, r, x);
   else hipLaunchKernelGGL(k_pupdate<3>, grid, blk, 0, ctx->stream, A, p, r, x);
   NQ_HIP(hipGetLastError());
@@ -524,7 +535,9 @@ int launch_cg_pupdate_pair(nq_ctx* ctx, const SpinorView& p_in, const SpinorView
   prof_begin(ctx, x.data ? "blas_xpupdate" : "blas_pupdate",
              (site_bytes(p_in) + site_bytes(p_out) + site_bytes(r) + xb) * (double)ctx->geo.Vh, &ev);
   const dim3 grid((unsigned)L.blocks), blk(L.threads);
-  if (p_in.ncomp == 12) hipLaunchKernelGGL(k_pupdate_pair<12>, grid, blk, 0, ctx->stream, A, p_in, p_out, r, x);
+  if (p_in.ncomp == 12 && fin != FIN_NONE)
+    hipLaunchKernelGGL((k_pupdate_pair<12, true>), grid, blk, 0, ctx->stream, A, p_in, p_out, r, x);
+  else if (p_in.ncomp == 12) hipLaunchKernelGGL(k_pupdate_pair<12>, grid, blk, 0, ctx->stream, A, p_in, p_out, r, x);
   else return fail(NQ_EINVAL, "pupdate pair: spincolor fields expected");
   NQ_HIP(hipGetLastError());
   prof_end(ctx, ev);

@@ -26,8 +26,9 @@ struct CgState {
   int iter, niter, done, reliable, nreliable, nan, mixed, pending;
   // done (bit 0) or reliable (bit 1) as raised by a finalisation that rides in a hop, whose
   // other workgroups read done and reliable: the CG tail and the reductions after that hop
-  // idle on either, and the p update that follows turns it into done and reliable, for
-  // every later launch.  launch_cg_commit clears it.
+  // idle on either, and the finalisation of |r|^2 that follows, or the p update in its
+  // place, turns it into done and reliable, for every later launch.  launch_cg_commit
+  // clears it.
   int stop;
   // paired x updates of the one-source mixed CG: xlag = the last p update left its
   // alpha p term to the next one; xstep = the coming p update applies both terms

@@ -374,8 +374,12 @@ __global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop(Geo g, i
 // 36.05 -> 35.73 ms), after every four otherwise (FP32 139 -> 132 us).
 // One right-hand side, neighbours staged in LDS (Stage): the workgroup's four
 // wavefronts cover 256 consecutive output sites (Shape W = 4, NRB = 1).
+// The FP64 write-only hop is held to two wavefronts per SIMD: with 12-real links its
+// registers would allow a third, which takes it from 240 to 243 us at 32^3x64.
 template <int SP, int LK, int MODE, int XP, int CLV = 0, int CP = kNT>
-__global__ void __launch_bounds__(256, (SP != SP_F64 ? 2 : 1)) k_tm_hop_lds(Geo g, int op, SpinorView out,
+__global__ void __attribute__((amdgpu_flat_work_group_size(1, 256),
+                               amdgpu_waves_per_eu(SP != SP_F64 ? 2 : 1, SP == SP_F64 && MODE == 0 ? 2 : 8)))
+k_tm_hop_lds(Geo g, int op, SpinorView out,
                                                                         SpinorView in, LinkView U, double anis_d,
                                                                         int use_anis, HopEpi epi, Shape S,
                                                                         int64_t nchunks, double* partial)

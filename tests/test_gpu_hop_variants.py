@@ -198,7 +198,7 @@ def test_persistent_hop_against_oracle(monkeypatch):
 # (NQ_LDS=0: they are not), and a batch runs the plain ones
 @pytest.mark.parametrize("prec", ["f16", "f16h", "f32"])
 def test_clover_with_streamed_links(prec, monkeypatch):
-    L, kappa, mu, n = (48, 24, 24, 24), 0.13, 0.05, 3
+    L, kappa, mu, n = (40, 24, 24, 24), 0.13, 0.05, 3
     conf = conf_of(L, 59, [1.0, 0, 0, 0])
     with nq.Ctx(L) as ctx:
         g = nq.Gauge(ctx, lx=conf)
