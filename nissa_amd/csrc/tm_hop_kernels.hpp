@@ -841,8 +841,8 @@ __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out
 // thirds of the VALU and with every slot waiting for its own loads.  Per right-hand side
 // and site this leaves 120 VALU instructions a slot (12 mixed adds, 12 scalings, 72
 // multiply-adds, 24 adds) of the 2159 a site took, at 224-247 registers and two wavefronts
-// per SIMD.  What bounds it now is the L1's rate of misses (TD busy 97 %, 15 B a cycle and
-// CU from L2).  Twelve right-hand sides: 24^3x48 235 -> 187 us (2.9 TB/s of compulsory
+// per SIMD.  What bounds it now is the L1's rate of misses (32^3x64: TD busy 99 %, 16 B a
+// cycle and CU from L2, 2.6 times the compulsory bytes).  Twelve right-hand sides: 24^3x48 235 -> 187 us (2.9 TB/s of compulsory
 // bytes), 32^3x64 692 -> 546, 16^3x32 48.5 -> 34.5; the z-tiled site order then takes
 // them to 177, 517 and 35.6.  Loading all stored elements before the first rebuild and
 // keeping the loop's loads unconditional matters: a load behind a branch makes every
