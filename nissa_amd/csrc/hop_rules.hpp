@@ -57,6 +57,23 @@ inline bool use_split(int64_t Vh, int sp, bool plain64, bool clover)
   return Vh < (int64_t(1) << bits);
 }
 
+// Neighbours staged in LDS in the register-blocked kernel, as far as the LDS holds two
+// workgroups or more (FP16 any RB, FP32 up to two, FP64 one right-hand side per wavefront).
+// The batched hop is bound by the L2->L1 path: twelve right-hand sides at 24^3x48, FP64
+// 825 -> 713 us, FP32 400 -> 308.  Where the blocks of all right-hand sides do not give
+// every CU more than one, the staging round trip only adds latency.  FP32 solves, not
+// staged / staged: 8^3x16, 2 sources 4.24 / 4.51 ms, 12 sources 6.30 / 6.68; 20x12^3, 2
+// sources 5.09 / 5.41, 5 sources 6.70 / 6.62, 8 sources 9.01 / 8.28; 32x12x14x12, 2 sources
+// 5.54 / 5.72, 3 sources 6.46 / 6.49; 20x16^3, 2 sources 6.26 / 6.01; 16x10x12^2, 5 sources
+// 5.98 / 6.36, 8 sources 7.08 / 7.31, 12 sources 9.58 / 8.97.  The staging is a template
+// parameter: as a branch it cost the launches that skip it 1.2 us of 10, and the FP16 tail
+// a wavefront per SIMD (five sources at 20^3x40: 61 -> 70 us).
+constexpr bool batch_stages(int sp, int rb) { return sp == SP_F16 || (sp == SP_F32 && rb <= 2) || (sp == SP_F64 && rb == 1); }
+inline bool stage_batch(int64_t Vh, int sp, int rb, int nr, int ncu)
+{
+  return batch_stages(sp, rb) && (Vh + 255) / 256 * nr > ncu;
+}
+
 // Kernel and cache policy of a hop that is not register-blocked.  xp: precision of the
 // other fields of the epilogue's tail; per_rhs: coefficients per right-hand side (a batch,
 // whose kernel does not depend on its size); lds: staging allowed.  keep: the default cache

@@ -759,7 +759,9 @@ __device__ __forceinline__ void hop_slot_rb(const Geo& g, const Site& s, uint32_
 // Multi-RHS hop for the sloppy precisions: wavefront w of a workgroup takes chunk
 // 4*cb + w and the RB right-hand sides of group rg (Shape: W = 4, NRB = 1, NR = NRG
 // = number of RB-groups).  Link traffic and link loads per right-hand side drop by RB.
-template <int SP, int LK, int MODE, int XP, int RB>
+// STG: the busy right-hand sides' records of the workgroup's 256 sites are staged in LDS
+// and the neighbours among those sites read from there (stage_batch).
+template <int SP, int LK, int MODE, int XP, int RB, bool STG>
 __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out, SpinorView in, LinkView U,
                                                    double anis_d, int use_anis, HopEpi epi, Shape S, int nr,
                                                    int64_t nchunks, double* partial)
@@ -771,15 +773,7 @@ __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out
 #pragma unroll
   for (int b = 0; b < RB; b++)
     if (b < nrb && !(epi.st && rhs_idle<MODE>(epi.st + r0 + b, epi.pred_reliable))) busy |= 1u << b;
-  // right-hand sides that idle here are skipped by the finalisation as well.
-  // The busy right-hand sides' records of the workgroup's 256 sites are staged in LDS and
-  // the neighbours among those sites read from there, as far as the LDS holds two
-  // workgroups or more (FP16 any RB, FP32 up to two, FP64 one right-hand side per
-  // wavefront).  The batched hop is bound by the L2->L1 path: twelve right-hand sides at
-  // 24^3x48, FP64 825 -> 713 us, FP32 400 -> 308.  On lattices of a few dozen blocks the
-  // staging round trip only adds latency (16x8^3, FP32: 8.0 -> 9.2 us), so they skip it.
-  constexpr bool STG = SP == SP_F16 || (SP == SP_F32 && RB <= 2) || (SP == SP_F64 && RB == 1);
-  const bool stage = STG && g.Vh >= 64 * kStageSites;
+  // right-hand sides that idle here are skipped by the finalisation as well
   __shared__ __attribute__((aligned(16))) char lds[STG ? RB * Stage<SP, 12>::BYTES : 16];
   const uint32_t e0 = (uint32_t)((m.chunk - (threadIdx.x >> 6)) * 64);
   if (!busy) {  // uniform over the workgroup (one right-hand-side group)
@@ -790,7 +784,7 @@ __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out
     }
     return;
   }
-  if (stage) {  // uniform over the launch
+  if constexpr (STG) {
 #pragma unroll
     for (int b = 0; b < RB; b++)
       if (b < nrb && ((busy >> b) & 1u))
@@ -798,7 +792,7 @@ __global__ void __launch_bounds__(256) k_tm_hop_rb(Geo g, int op, SpinorView out
                            e0 + threadIdx.x < (uint64_t)g.Vh, (int)threadIdx.x, r0 + b);
     __syncthreads();
   }
-  const char* lp = stage ? lds : nullptr;
+  const char* lp = STG ? lds : nullptr;
   const uint32_t e = m.e;
   cx<R> o[RB][12];
 #pragma unroll
@@ -970,11 +964,21 @@ static int launch_rb(nq_ctx* ctx, int RB, int op, const SpinorView& out, const S
   sh.NRG = sh.NR = (nr + RB - 1) / RB;
   const int64_t nchunks = (g.Vh + 63) / 64;
   const dim3 grid((unsigned)((nchunks + 3) / 4 * sh.NRG)), blk(256);
+#define NQ_RB(N)                                                                                                      \
+  do {                                                                                                               \
+    if (stage_batch(g.Vh, SP, N, nr, ctx->ncu))                                                                                  \
+      NQ_HOP_LAUNCH((k_tm_hop_rb<SP, LK, MODE, XP, N, batch_stages(SP, N)>), grid, blk, g, op, out, in, U, anis, ua,  \
+                    epi, sh, nr, nchunks, ctx->partial);                                                             \
+    else                                                                                                             \
+      NQ_HOP_LAUNCH((k_tm_hop_rb<SP, LK, MODE, XP, N, false>), grid, blk, g, op, out, in, U, anis, ua, epi, sh, nr,   \
+                    nchunks, ctx->partial);                                                                          \
+  } while (0)
   switch (RB) {
-  case 1: NQ_HOP_LAUNCH((k_tm_hop_rb<SP, LK, MODE, XP, 1>), grid, blk, g, op, out, in, U, anis, ua, epi, sh, nr, nchunks, ctx->partial); break;
-  case 2: NQ_HOP_LAUNCH((k_tm_hop_rb<SP, LK, MODE, XP, 2>), grid, blk, g, op, out, in, U, anis, ua, epi, sh, nr, nchunks, ctx->partial); break;
-  default: NQ_HOP_LAUNCH((k_tm_hop_rb<SP, LK, MODE, XP, 4>), grid, blk, g, op, out, in, U, anis, ua, epi, sh, nr, nchunks, ctx->partial); break;
+  case 1: NQ_RB(1); break;
+  case 2: NQ_RB(2); break;
+  default: NQ_RB(4); break;
   }
+#undef NQ_RB
   NQ_HIP(hipGetLastError());
   return NQ_OK;
 }

@@ -222,3 +222,21 @@ def test_clover_with_streamed_links(prec, monkeypatch):
         one = [ctx.field(nq.SPINCOLOR, nq.LX)]
         nq.tmclov_solve_eoprec_multi(ctx, g, cl, kappa, mu, 1000, 1e-14, one, src[2:], prec=prec)
         assert np.array_equal(one[0].download(), batch[2])
+
+
+# 110 blocks: staged from three right-hand sides up on 256 CUs; 40 blocks, from seven
+@pytest.mark.parametrize("L,nr", [((28, 12, 12, 14), 3), ((10, 12, 12, 14), 7)])
+@pytest.mark.parametrize("prec", ["f64", "f32", "f16"])
+def test_staged_batch_same_bits_alone(L, nr, prec, monkeypatch):
+    monkeypatch.setenv("NQ_TUNE", "0")  # the register-blocked kernel, also for FP16
+    conf = conf_of(L, 60, [1.0, 0, 0, 0])
+    with nq.Ctx(L) as ctx:
+        g = nq.Gauge(ctx, lx=conf)
+        src = [ctx.field(nq.SPINCOLOR, nq.LX, nq.source_lx(L, 65 + i)) for i in range(nr)]
+        sol = [ctx.field(nq.SPINCOLOR, nq.LX) for _ in src]
+        out = []
+        for n in (nr, 1):
+            res = nq.tm_solve_eoprec_multi(ctx, g, 0.16, [0.05] * n, 1000, 1e-14, sol[:n], src[:n], prec=prec)
+            assert all(r["rc"] == nq.NQ_OK for r in res), res
+            out.append(sol[0].download())
+        assert np.array_equal(out[0], out[1])

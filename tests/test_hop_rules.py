@@ -34,16 +34,42 @@ LINK = {0: 144, 1: 72, 2: 48, 3: 24, 4: 96}  # bytes of a link
 PLAIN, LDS, SPLIT = 0, 1, 2
 
 
-@pytest.fixture(scope="module")
-def routes(tmp_path_factory):
+SMALL = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "hop_rules.hpp"
+using namespace nq;
+
+int main()
+{
+  for (int64_t blocks : {1, 16, 45, 68, 110, 126, 160, 256, 375, 625, 1296, 4096})
+    for (int nr = 2; nr <= 16; nr++)
+      for (int sp : {SP_F64, SP_F32, SP_F16})
+        std::printf("%d %d %d %d %d %d\n", (int)blocks, nr, sp, stage_batch(256 * blocks, sp, 1, nr, 256),
+                    stage_batch(256 * blocks, sp, 4, nr, 256), 0);
+}
+"""
+
+
+def numbers(tmp_path_factory, source):
     if shutil.which("g++") is None:
         pytest.skip("no host C++ compiler")
     d = tmp_path_factory.mktemp("rules")
-    (d / "t.cpp").write_text(SRC)
+    (d / "t.cpp").write_text(source)
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Wextra", "-Werror", "-I", CSRC, str(d / "t.cpp"), "-o", str(d / "t")],
                    check=True)
     out = subprocess.run([str(d / "t")], check=True, capture_output=True, text=True).stdout
     return [tuple(int(v) for v in l.split()) for l in out.splitlines()]
+
+
+@pytest.fixture(scope="module")
+def routes(tmp_path_factory):
+    return numbers(tmp_path_factory, SRC)
+
+
+@pytest.fixture(scope="module")
+def small(tmp_path_factory):
+    return numbers(tmp_path_factory, SMALL)
 
 
 def test_one_policy_for_every_kernel(routes):
@@ -65,3 +91,10 @@ def test_staged_hops_that_keep_their_links(routes):
     the default policy happens in FP64 clover hops and batched residuals only."""
     kept = {(sp, clover, per_rhs) for sp, lk, xp, clover, per_rhs, Vh, kernel, keep in routes if kernel == LDS and keep}
     assert kept == {(F64, 1, 0), (F64, 0, 1)}
+
+
+def test_batches_stage_where_they_fill_the_card(small):
+    """A staged batch has more blocks, over all of its right-hand sides, than there are CUs."""
+    for blocks, nr, sp, rb1, rb4, _ in (l for l in small if len(l) == 6):
+        assert rb1 == (blocks * nr > 256)
+        assert rb4 == (rb1 and sp == F16)  # LDS for four right-hand sides: FP16 only
