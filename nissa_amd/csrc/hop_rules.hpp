@@ -101,4 +101,23 @@ inline HopRoute hop_route(int64_t Vh, int sp, int lk, int xp, bool clover, int n
 // and, in a batch, the residual (mode 3).
 constexpr bool hop_lds_keeps(int sp, int mode, bool clover) { return sp == SP_F64 && (mode == 3 || clover); }
 
+// Right-hand sides per wavefront of the staggered hops for nr > 1: 6 for FP32 batches of
+// five or more, else 4, and fewer on a lattice whose 256-site blocks then give less than two
+// workgroups per CU.  Multi-shift CG, with 4 or 6 -> with the block taken: 16^3x32, 4
+// sources, 10 shifts, FP32 51.5 -> 46.9 ms, FP64 42.6 -> 39.1; 26x14^3, 3 x 9, FP32 35.6 ->
+// 30.5; 16x8^3, 4 x 12, 33.1 -> 24.4; 20x10^3, 2 x 8, FP64 17.2 -> 14.5.  20^3x40, 4 x 10,
+// FP64 keeps 4: 102.5 (2: 101.1, 1: 126.5).
+// One per wavefront re-reads the links for every source, and pays only while the blocks of
+// all sources leave the card that empty: one block (FP64) or two (FP32) per CU.  RB = 1 / 2:
+// FP64 28x12^2x14, 2 sources 17.6 / 19.0 ms, 3 sources 23.7 / 20.3; 20x16^3, 2 sources 16.5 /
+// 14.0, 4 sources 25.7 / 20.1; 24x20^3, 2 sources 31.8 / 26.3; FP32 20x16^3, 2 sources 19.8 /
+// 21.0; 26x16^3, 4 sources 37.8 / 34.4; 24x20^3, 2 sources 28.6 / 27.2.
+inline int st_block(int64_t Vh, int nr, int sp, int ncu)
+{
+  const int64_t nblk = (Vh + 255) / 256, alone = (sp == SP_F64 ? 1 : 2) * ncu;
+  int v = sp == SP_F32 && nr >= 5 ? 6 : 4;
+  while (v > 1 && nblk * ((nr + v - 1) / v) < 2 * ncu && (v > 2 || nblk * nr <= alone)) v = v > 4 ? 4 : v / 2;
+  return v;
+}
+
 }  // namespace nq

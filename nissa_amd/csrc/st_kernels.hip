@@ -822,12 +822,7 @@ static double lbytes(int lk) { return lk == LK_F64_18 ? 144.0 : 72.0; }
 // multi-shift hop 1214 against 1245 us with RB = 4; the 16-system refinement CG's
 // fused tail 511 against 534-557 us with RB = 8 or 4); else 4 (FP64: RB = 6 takes
 // 208 VGPRs and 72 KB of LDS, two wavefronts per SIMD, and measured 2 % slower).
-// A lattice with too few 256-site blocks for two workgroups per CU takes fewer per
-// wavefront, for more workgroups.  Multi-shift CG with the block above -> with the one
-// the rule takes: 16^3x32, 4 sources, 10 shifts, FP32 51.5 -> 46.9 ms, FP64 42.6 -> 39.1
-// (RB = 1: 58.1, 51.0); 26x14^3, 3 x 9, FP32 35.6 -> 30.5; 16x8^3, 4 x 12, 33.1 -> 24.4;
-// 20x10^3, 2 x 8, FP64 17.2 -> 14.5.  20^3x40, 4 x 10, FP64 keeps 4: 102.5 (2: 101.1,
-// 1: 126.5).
+// A lattice with too few 256-site blocks takes fewer per wavefront (st_block).
 // NQ_ST_RB = 1, 2, 4, 6 or 8 (8: FP32 only) overrides; every choice gives the same
 // bits.  The launch shape for RB: W = 4 chunks per workgroup, one RB group per
 // wavefront.
@@ -835,11 +830,7 @@ static int st_rb(const nq_ctx* ctx, int nr, int sp)
 {
   if (nr <= 1) return 1;
   const char* e = getenv("NQ_ST_RB");
-  int v = e ? atoi(e) : (sp == SP_F32 && nr >= 5 ? 6 : 4);
-  if (!e) {
-    const int64_t nblk = (ctx->geo.Vh + kStageSites - 1) / kStageSites;
-    while (v > 1 && nblk * ((nr + v - 1) / v) < 2 * ctx->ncu) v = v > 4 ? 4 : v / 2;
-  }
+  const int v = e ? atoi(e) : st_block(ctx->geo.Vh, nr, sp, ctx->ncu);
   if (v == 8) return sp == SP_F32 ? 8 : 4;
   return v == 1 || v == 2 || v == 6 ? v : 4;
 }

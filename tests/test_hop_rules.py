@@ -46,7 +46,7 @@ int main()
     for (int nr = 2; nr <= 16; nr++)
       for (int sp : {SP_F64, SP_F32, SP_F16})
         std::printf("%d %d %d %d %d %d\n", (int)blocks, nr, sp, stage_batch(256 * blocks, sp, 1, nr, 256),
-                    stage_batch(256 * blocks, sp, 4, nr, 256), 0);
+                    stage_batch(256 * blocks, sp, 4, nr, 256), sp == SP_F16 ? 0 : st_block(256 * blocks, nr, sp, 256));
 }
 """
 
@@ -98,3 +98,19 @@ def test_batches_stage_where_they_fill_the_card(small):
     for blocks, nr, sp, rb1, rb4, _ in (l for l in small if len(l) == 6):
         assert rb1 == (blocks * nr > 256)
         assert rb4 == (rb1 and sp == F16)  # LDS for four right-hand sides: FP16 only
+
+
+def test_staggered_block_shrinks_with_the_lattice(small):
+    """One source per wavefront only while all blocks of all sources leave the card near
+    empty; the block never shrinks on the way to a larger lattice."""
+    last = {}
+    for blocks, nr, sp, _, _, v in (l for l in small if len(l) == 6):
+        if sp == F16:
+            continue
+        full = 6 if sp == F32 and nr >= 5 else 4
+        assert v in (1, 2, 4, 6) and v <= full and v >= last.get((nr, sp), 1)
+        last[nr, sp] = v
+        if v == 1:
+            assert blocks * nr <= (256 if sp == F64 else 512)
+        if blocks >= 512:
+            assert v == full
