@@ -247,8 +247,8 @@ Geo make_geo(int T, int LX, int LY, int LZ, int tbmax, int tx, int ty)
   g.TX = tx; g.logTX = lg(tx); g.NXT = LX / tx;
   g.TY = ty; g.logTY = lg(ty); g.NYT = LY / ty;
   // pairs of z rows: with the 4 x 2 patch, 256 consecutive sites of a 64-slice t tile are
-  // a 2 x 2 x 2 cell of rows (NQ_ZTILE overrides; a power of two up to 16)
-  int tz = 2;
+  // a 2 x 2 x 2 cell of rows (z_tile; NQ_ZTILE overrides; a power of two up to 16)
+  int tz = z_tile(T, g.Vh);
   if (const char* ez = getenv("NQ_ZTILE")) tz = atoi(ez);
   if (!pow2(tz)) tz = 1;
   while (LZ % tz) tz /= 2;

@@ -120,4 +120,15 @@ inline int st_block(int64_t Vh, int nr, int sp, int ncu)
   return v;
 }
 
+// Rows of a z tile of the site order (halved until it divides the extent).  Two, which with
+// the 4 x 2 patch make 256 consecutive sites of a 64-slice t tile a 2 x 2 x 2 cell of rows.
+// Eight below 2^16 sites per parity, where a wavefront covers many rows: its x and y
+// neighbours are then all inside the workgroup or all outside it, and a load is not split in
+// two by the branch (two / eight rows: two FP32 sources on 8^4 4.26 / 3.93 ms, three at
+// 24x12^2x16 6.07 / 5.75; FP64 shifts, one source, 16x6^2x8 13.3 / 12.8; 16^3x32, three FP32
+// sources, 9.30 / 9.66).  Four where the t extent is no multiple of eight and the rows cut
+// across wavefronts (two / four: two FP16 sources at 30x24^3 15.8 / 15.5 ms, six 36.6 / 35.6;
+// FP64 at 22x26x28^2 22.5 / 22.2; 24^4 and 32x20^3 equal or worse).
+inline int z_tile(int T, int64_t Vh) { return Vh < (int64_t(1) << 16) ? 8 : (T % 8 ? 4 : 2); }
+
 }  // namespace nq

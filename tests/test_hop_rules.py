@@ -47,6 +47,8 @@ int main()
       for (int sp : {SP_F64, SP_F32, SP_F16})
         std::printf("%d %d %d %d %d %d\n", (int)blocks, nr, sp, stage_batch(256 * blocks, sp, 1, nr, 256),
                     stage_batch(256 * blocks, sp, 4, nr, 256), sp == SP_F16 ? 0 : st_block(256 * blocks, nr, sp, 256));
+  for (int T : {4, 8, 16, 22, 30, 32, 36, 48, 64})
+    for (int64_t Vh : {8, 65535, 65536, 1048576}) std::printf("%d %d %d\n", T, (int)Vh, z_tile(T, Vh));
 }
 """
 
@@ -114,3 +116,8 @@ def test_staggered_block_shrinks_with_the_lattice(small):
             assert blocks * nr <= (256 if sp == F64 else 512)
         if blocks >= 512:
             assert v == full
+
+
+def test_z_tile(small):
+    for T, Vh, z in (l for l in small if len(l) == 3):
+        assert z == (8 if Vh < 65536 else 4 if T % 8 else 2)
